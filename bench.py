@@ -59,9 +59,7 @@ WORKLOAD = SUPERBLOCKS["hubbard_L64_m400"][0]
 PROFILE_EVERY = 16
 PEAK_HBM_GBS = 8000.0
 PEAK_FP64_MFMA_TFLOPS = 78.6   # MI355X dense FP64 matrix peak
-KRON_VARIANTS = ["FP64 vector units, 64 x 64 tiles", "FP64 MFMA, 64 x 64 tiles", "FP64 MFMA, 128 x 128 tiles",
-                 "FP64 MFMA, 64 x 128 tiles", "FP64 MFMA, 128 x 64 tiles", "FP64 MFMA, 64 x 64 tiles, k-slabs of 32",
-                 "FP64 MFMA, 64 x 64 tiles, four wavefronts per SIMD", "FP64 MFMA, 128 x 128 tiles, two wavefronts per SIMD"]
+KRON_FORMS = {0: "16 x 16 output tiles", 1: "output tiles by size", 2: "32 x 32 output tiles"}
 SPMV_FORMATS = [("CSR", "k_apply<CsrRows<double>> (CSR SpMV + fused Lanczos/CG epilogue)"),
                 ("value dictionary", "k_apply<DictRows> (value-dictionary CRS SpMV + fused Lanczos/CG epilogue)"),
                 ("delta columns", "k_apply<DeltaRows<double>> (delta-column CRS SpMV + fused Lanczos/CG epilogue)"),
@@ -886,7 +884,6 @@ def run_kron(D, L, name, steps, warmup, lan_type=0, profile=True):
     avg_s = ms.value / 1e3 / max(launches.value, 1)
     fl = flops.value / max(launches.value, 1)
     achieved = fl / avg_s / 1e12 if avg_s > 0 else 0.0
-    v = variant % len(KRON_VARIANTS)
     return {
         "value": round(steps / total, 4),
         "ms_per_step": round(total / steps * 1e3, 3),
@@ -904,13 +901,12 @@ def run_kron(D, L, name, steps, warmup, lan_type=0, profile=True):
             "max_gs_error": float(max(gerr)),
             "lanczos_steps": int(np.median(lan)),
             "cg_steps": int(np.median(cg)),
-            "product_kernel": {"variant": variant, "form": KRON_VARIANTS[v],
-                               "xcd_contiguous_tiles": variant >= len(KRON_VARIANTS)},
+            "product_kernel": {"variant": variant, "form": KRON_FORMS.get(variant, KRON_FORMS[1])},
         },
         "roofline": {
             "bound": "mfma",
-            "kernel": "k_kron_tile<64, 64, true> (dense sector products M_L X and X M_R^T on v_mfma_f64_16x16x4)"
-                      if v == 1 else f"k_kron_tile ({KRON_VARIANTS[v]})",
+            "kernel": "k_kron (M_L X + X M_R^T per output tile on v_mfma_f64_16x16x4, with the coupling terms and "
+                      "the solver's epilogue)",
             "achieved": round(achieved, 2),
             "peak": PEAK_FP64_MFMA_TFLOPS,
             "unit": "TFLOP/s",
@@ -919,8 +915,8 @@ def run_kron(D, L, name, steps, warmup, lan_type=0, profile=True):
             "alg_flops_per_launch": int(fl),
             "avg_launch_us": round(avg_s * 1e6, 2),
             "launches": int(launches.value),
-            "launches_sampled": f"1 in {PROFILE_EVERY} of the timed solves' products, HIP events on the library "
-                                "stream around the dense-product kernel",
+            "launches_sampled": f"1 in {PROFILE_EVERY} of the timed solves' products that always run in full, HIP "
+                                "events on the library stream around the product kernel",
         },
     }
 

@@ -688,13 +688,10 @@ int ground_state_op(const Operator &op, const dmrgx_matrix *A, const dmrgx_solve
       } else {   // the 1 x 1 operator applied to 1
         const double one = 1.0;
         v.up(&one);
-        op.kron->product(v.d.p, st);
+        DevBuf<double> hv(1);
+        launch_spmv(op, v.d.p, hv.p, st);
         HIPCHK(hipStreamSynchronize(st));   // the library's streams do not block on the null stream
-        double hl, hc;
-        HIPCHK(hipMemcpy(&h, op.kron->z.p, sizeof(double), hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(&hl, op.kron->zl.p, sizeof(double), hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(&hc, op.kron->zc.p, sizeof(double), hipMemcpyDeviceToHost));
-        h = (h + hl) + hc;
+        HIPCHK(hipMemcpy(&h, hv.p, sizeof(double), hipMemcpyDeviceToHost));
       }
       out.eig = h;
       const double one = 1.0;

@@ -860,50 +860,83 @@ struct KronSector {
   int64_t ml, mr;     // offsets of the sector's M_L and M_R in KronDev::ML / MR
   int32_t a0, b0;     // first of its LLLR / RRRL states in the flat state lists
 };
-// Tile shapes of the dense sector products and the product kernels over them: variant 0
-// the FP64 vector form on 64 x 64 tiles, 1-4 the FP64 matrix cores on 64 x 64, 128 x 128,
-// 64 x 128 and 128 x 64 tiles, 5 the matrix cores on 64 x 64 tiles with k-slabs of 32, 6 as 1
-// held to four wavefronts per SIMD, 7 as 2 held to two.
-constexpr int kKronShapes = 4;
-inline constexpr int kKronTM[kKronShapes] = {64, 128, 64, 128};
-inline constexpr int kKronTN[kKronShapes] = {64, 128, 128, 64};
-constexpr int kKronVariants = 8;
-constexpr int kKronDefault = 1;   // 64 x 64 tiles, FP64 matrix cores, default occupancy, no XCD mapping
-inline constexpr int kKronShape[kKronVariants] = {0, 0, 1, 2, 3, 0, 0, 1};
+// First k of slab s of a product whose k runs over dim states: slabs of 16, the last one shifted
+// back to end with the range.
+__host__ __device__ inline int32_t kron_slab(int32_t s, int32_t dim) {
+  const int32_t last = dim > 16 ? dim - 16 : 0;
+  return 16 * s < last ? 16 * s : last;
+}
+// Place of element (r, k) of a dim x dim sector matrix M_L or M_R: 16 rows by one slab after
+// another, block rows one after another, a block in the order in which a wavefront's lanes take
+// it as a matrix-instruction fragment (lane 16 (p / 4) + r mod 16 holds places p mod 4 = 0 .. 3 of the
+// slab; all lanes' first pairs, then all second pairs).  An element is stored once: a k that the
+// shifted last slab repeats is zero there, as is everything outside the matrix.
+__host__ __device__ inline int64_t kron_at(int32_t r, int32_t k, int32_t dim) {
+  const int32_t ns = (dim + 15) >> 4, s = k >> 4, p = k - kron_slab(s, dim);
+  const int32_t lane = 16 * (p >> 2) + (r & 15);
+  return ((int64_t)(r >> 4) * ns + s) * 256 + ((p & 2) ? 128 : 0) + 2 * lane + (p & 1);
+}
+// An output tile of the product kernel: its first row and column within its sector, and what the
+// kernel needs of the sector (one load before the first operands').
+struct KronTile {
+  int64_t off, ml, mr;
+  int32_t da, db, a0, b0, r0, c0;
+  KronTile() = default;
+  KronTile(const KronSector &s, int32_t r, int32_t c)
+      : off(s.off), ml(s.ml), mr(s.mr), da(s.da), db(s.db), a0(s.a0), b0(s.b0), r0(r), c0(c) {}
+};
+// A coupling term on one half: what the term's operator does to a state.  Left: at = the
+// vector index of the target state's row (first RRRL state); right: at = the target state's
+// place within its sector; -1 without a target.  c: the coefficient (sign rule, operator
+// element, on the left the term's factor).
+struct KronMap {
+  double c;
+  int32_t at, pad;
+};
+// What the product kernel (kron_tile.h) reads.
+struct KronView {
+  const KronTile *tiles;
+  const double *ML, *MR;
+  int32_t ncross, na, nb;
+  const KronMap *lmap, *rmap;   // [term][flat state]
+  const double *zc;             // coupling terms applied beforehand (KronDev::general), or null
+};
+// Output tiles of the product kernel, by shape.
+constexpr int kKronShapes = 2;
+inline constexpr int kKronTile[kKronShapes] = {16, 32};
+// Product kernels a caller can choose (dmrgx_kron_set_kernel): 0 and 2 fix the shape 16 x 16 and
+// 32 x 32, the default and every other number take it by size (kron_shape_rule).
+constexpr int kKronVariants = 16;
+constexpr int kKronDefault = 1;
 struct KronDev {
   int32_t n = 0, nsec = 0, ncross = 0, na = 0, nb = 0;
-  int32_t ntiles[kKronShapes] = {0, 0, 0, 0};
-  int variant = kKronDefault;             // product kernel (kKronShape of it picks the tiles)
-  int xcd = 0;                            // 1: consecutive tiles to the blocks of one XCD
+  int32_t ntiles[kKronShapes] = {0, 0};
+  int variant = kKronDefault;             // product kernel
+  int rule = 0;                           // the shape that kKronDefault takes
   const dmrgx_superblock *sb = nullptr;   // borrowed: basis, inverse, operators, term list
   std::vector<KronSector> hsec;
   DevBuf<KronSector> sec;
-  DevBuf<double> ML, MR;                  // dense sector blocks, row-major
-  DevBuf<int32_t> tiles[kKronShapes];     // per shape: (sector, tile row, tile column, left/right)
-  DevBuf<int32_t> cross;                  // indices of the coupling terms in the term list
-  // per coupling term: its factor, and the LLLR / RRRL states each state reaches with the
-  // term's operator on that half, with coefficients (k_kron_cross)
+  DevBuf<double> ML, MR;                  // dense sector blocks (kron_at)
+  DevBuf<KronTile> tiles[kKronShapes];
+  DevBuf<KronMap> lmap, rmap;             // per coupling term and state
+  // The general form of the coupling terms, kept when some state has more than one target
+  // under a term (operators of a block, not of a site): per term its factor, and the LLLR / RRRL
+  // states each state reaches with the term's operator on that half (k_kron_cross, into zc
+  // before the product kernel).
+  bool general = false;
   DevBuf<double> ct, lval, rval;
   DevBuf<int32_t> lptr, lidx, rptr, ridx;
   // flat LLLR / RRRL state of (LL d + LR) / (RR d + RL) (-1: none) and each flat state's sector
   DevBuf<int32_t> aidx, bidx, asec, bsec;
-  mutable DevBuf<double> z, zl, zc;       // H x of the last product is (z + zl) + zc: right, left, coupling
-  mutable hipStream_t side = nullptr;     // the coupling terms' stream (default priority)
-  mutable hipEvent_t fork = nullptr, join = nullptr;
-  KronDev() = default;
-  KronDev(const KronDev &) = delete;
-  KronDev &operator=(const KronDev &) = delete;
-  ~KronDev() {
-    if (side) {
-      (void)hipStreamSynchronize(side);
-      (void)hipStreamDestroy(side);
-    }
-    if (fork) (void)hipEventDestroy(fork);
-    if (join) (void)hipEventDestroy(join);
-  }
+  DevBuf<double> zc;
   double flops = 0.0;                     // of the two dense products per H x
-  // z = H x on stream s
-  void product(const double *x, hipStream_t s) const;
+  int shape() const;
+  KronView view() const {
+    return KronView{tiles[shape()].p, ML.p, MR.p, general ? 0 : ncross, na, nb, lmap.p, rmap.p,
+                    general ? zc.p : nullptr};
+  }
+  // the general form's coupling terms of x into zc
+  void cross(const double *x, hipStream_t s) const;
 };
 
 // The operator a solver applies: an assembled full CSR, the matrix-free OBC form, or the

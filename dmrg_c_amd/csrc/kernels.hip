@@ -184,6 +184,16 @@ struct LateBegin : std::false_type {};
 template <class E>
 struct LateBegin<E, std::void_t<decltype(E::kLateBegin)>> : std::bool_constant<E::kLateBegin> {};
 
+// The epilogue's prefetched values (LateBegin), or nothing.
+template <class E, class = void>
+struct PreOf {
+  using type = int;
+};
+template <class E>
+struct PreOf<E, std::void_t<typename E::Pre>> {
+  using type = typename E::Pre;
+};
+
 template <int G, class Rows, class Epi>
 __global__ __launch_bounds__(kBlock) void k_apply(int32_t n, Rows rows, const double *__restrict__ x, Epi epi,
                                                   double *partial, int xcd) {
@@ -222,6 +232,14 @@ __global__ __launch_bounds__(kBlock) void k_apply(int32_t n, Rows rows, const do
   }
   if constexpr (Epi::kReduce) block_partial_to(c, partial + lb);
 }
+
+}  // namespace
+}  // namespace dmrgx
+
+#include "kron_tile.h"
+
+namespace dmrgx {
+namespace {
 
 struct EpiPlain {
   double *y;
@@ -575,17 +593,37 @@ int apply_sell(const Operator &op, bool fp32, const double *x, const Epi &epi, R
   throw Failure(DMRGX_ERR_ARG, "sliced form needs 1, 2 or 4 lanes per row");
 }
 
-// Rows of a product computed beforehand (the Kronecker form writes H x into z): one lane per
-// row returns z[r], so that the solvers' fused epilogues run on it unchanged.
-struct PreRows {
-  const double *z, *zl, *zc;   // the product is (z[r] + zl[r]) + zc[r]
-  static constexpr bool kTimed = false;
-  double alg_bytes(int32_t) const { return 0.0; }
-  template <int G>
-  __device__ __forceinline__ double lane_sum(int32_t r, int lane, const double *__restrict__) const {
-    return lane == 0 ? (z[r] + zl[r]) + zc[r] : 0.0;
+// The Kronecker form's product with its epilogue; returns the number of partials.
+template <class Epi>
+int apply_kron(const KronDev &K, const double *x, const Epi &epi, Reduce *R, hipStream_t s, bool fin) {
+  const int shape = K.shape(), nt = K.ntiles[shape];
+  if (nt == 0) return 0;
+  double *part = nullptr;
+  if (Epi::kReduce) {
+    R->ensure(nt);
+    part = R->partial.p;
   }
-};
+  K.cross(x, s);
+  // live timing (dmrgx_profile_begin_sampled): the dense products' floating-point operations
+  // where the CRS products count bytes
+  Context &C = ctx();
+  std::pair<hipEvent_t, hipEvent_t> *ev = nullptr;
+  if (!MaySkip<Epi>::value && C.prof_take()) {
+    ev = C.prof_slot();
+    HIPCHK(hipEventRecord(ev->first, s));
+    C.prof_bytes += K.flops;
+  }
+  const KronView v = K.view();
+  if (shape == 0) k_kron<1><<<nt, kBlock, 0, s>>>(v, x, epi, part);
+  else k_kron<2><<<nt, kBlock, 0, s>>>(v, x, epi, part);
+  HIPCHK(hipGetLastError());
+  if (ev) HIPCHK(hipEventRecord(ev->second, s));
+  if (Epi::kReduce && fin) {
+    k_finish<Epi><<<1, kBlock, 0, s>>>(epi, part, nt);
+    HIPCHK(hipGetLastError());
+  }
+  return nt;
+}
 
 template <class Epi>
 int apply_op(const Operator &op, bool fp32, const double *x, const Epi &epi, Reduce *R, hipStream_t s,
@@ -593,8 +631,7 @@ int apply_op(const Operator &op, bool fp32, const double *x, const Epi &epi, Red
   if (op.obc) return apply_rows(op.n, op.lanes, op.grid, op.obc->rows(), x, epi, R, s, 0, fin);
   if (op.kron) {
     if (fp32) throw Failure(DMRGX_ERR_ARG, "the Kronecker form has no FP32 values");
-    op.kron->product(x, s);
-    return apply_rows(op.n, 1, op.grid, PreRows{op.kron->z.p, op.kron->zl.p, op.kron->zc.p}, x, epi, R, s, 0, fin);
+    return apply_kron(*op.kron, x, epi, R, s, fin);
   }
   const int fmt = load_format(op.load);
   if (fmt == kFmtSellIdx && ensure_sell(*op.A, op.lanes, false)) {

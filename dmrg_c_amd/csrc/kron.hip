@@ -16,11 +16,10 @@
 // row by row from the term list through the superblock inverse, as the matrix-free product of
 // dmrg/DMRG_MATRIX_VECTOR_PRODUCT_OBC.c:18-83 applies its M_LRRL.
 //
-// A product is two kernels: the coupling terms write z row by row, then one LDS-tiled FP64
-// kernel whose workgroups each take a 64 x 64 tile of M_L X (written to zl) or of X M_R^T
-// (added to z); the solvers' epilogues read z + zl.  The sums are in an order of
-// their own (the CRS sums every term's contributions to an entry first), so results agree
-// with the CRS product to rounding.
+// A product is one kernel (kron_tile.h): each workgroup computes an output tile of both dense
+// products on the FP64 matrix cores, adds the coupling terms and runs the solver's epilogue.
+// The sums are in an order of their own (the CRS sums every term's contributions to an
+// entry first), so results agree with the CRS product to rounding.
 
 #include <hip/hip_runtime.h>
 
@@ -54,7 +53,7 @@ __global__ __launch_bounds__(256) void k_kron_left(KronBuild kb, const DTerm *te
   const int s = kb.asec[i];
   const KronSector S = kb.sec[s];
   const int32_t ap = i - S.a0;
-  double *row = ML + S.ml + (int64_t)ap * S.da;
+  double *M = ML + S.ml;
   const int q[4] = {kb.aLL[i], kb.aLR[i], 0, 0};
   for (int u = 0; u < nt; u++) {
     const DTerm t = terms[ids[u]];
@@ -67,7 +66,7 @@ __global__ __launch_bounds__(256) void k_kron_left(KronBuild kb, const DTerm *te
       const double p1 = sc * a.val[i1];
       if (t.s2 < 0) {
         const int32_t c = kb.aidx[qq[0] * kb.d + qq[1]];
-        if (c >= 0 && kb.asec[c] == s && fabs(p1) > 1.0e-15) row[c - S.a0] += p1;
+        if (c >= 0 && kb.asec[c] == s && fabs(p1) > 1.0e-15) M[kron_at(ap, c - S.a0, S.da)] += p1;
         continue;
       }
       const DOp b = ops[t.op2];
@@ -76,7 +75,7 @@ __global__ __launch_bounds__(256) void k_kron_left(KronBuild kb, const DTerm *te
         qq[t.s2] = b.col[i2];
         const double p = p1 * b.val[i2];
         const int32_t c = kb.aidx[qq[0] * kb.d + qq[1]];
-        if (c >= 0 && kb.asec[c] == s && fabs(p) > 1.0e-15) row[c - S.a0] += p;
+        if (c >= 0 && kb.asec[c] == s && fabs(p) > 1.0e-15) M[kron_at(ap, c - S.a0, S.da)] += p;
       }
     }
   }
@@ -90,7 +89,7 @@ __global__ __launch_bounds__(256) void k_kron_right(KronBuild kb, const DTerm *t
   const int s = kb.bsec[i];
   const KronSector S = kb.sec[s];
   const int32_t bp = i - S.b0;
-  double *row = MR + S.mr + (int64_t)bp * S.db;
+  double *M = MR + S.mr;
   const int q[4] = {0, 0, kb.bRR[i], kb.bRL[i]};
   for (int u = 0; u < nt; u++) {
     const DTerm t = terms[ids[u]];
@@ -103,7 +102,7 @@ __global__ __launch_bounds__(256) void k_kron_right(KronBuild kb, const DTerm *t
       const double p1 = sc * a.val[i1];
       if (t.s2 < 0) {
         const int32_t c = kb.bidx[qq[2] * kb.d + qq[3]];
-        if (c >= 0 && kb.bsec[c] == s && fabs(p1) > 1.0e-15) row[c - S.b0] += p1;
+        if (c >= 0 && kb.bsec[c] == s && fabs(p1) > 1.0e-15) M[kron_at(bp, c - S.b0, S.db)] += p1;
         continue;
       }
       const DOp b = ops[t.op2];
@@ -112,22 +111,22 @@ __global__ __launch_bounds__(256) void k_kron_right(KronBuild kb, const DTerm *t
         qq[t.s2] = b.col[i2];
         const double p = p1 * b.val[i2];
         const int32_t c = kb.bidx[qq[2] * kb.d + qq[3]];
-        if (c >= 0 && kb.bsec[c] == s && fabs(p) > 1.0e-15) row[c - S.b0] += p;
+        if (c >= 0 && kb.bsec[c] == s && fabs(p) > 1.0e-15) M[kron_at(bp, c - S.b0, S.db)] += p;
       }
     }
   }
 }
 
-// z = coupling terms applied to x.  A coupling term has one operator on each half (op1 on
-// LL or LR, op2 on RR or RL) and a sign that is a product of a factor of the row's LLLR state
-// and one of its RRRL state, so per term the builder lists, for every LLLR state a', the
-// states a it reaches with op1 and their coefficients (left parity sign x op1 value), and
-// likewise for every RRRL state b' (right parity sign x op2 value); the term's own factor is
-// its coefficient times the sign rule's constant.  One workgroup per LLLR state a' of the
-// output, its threads over the sector's RRRL states b': for each term (in term order), op1
-// entry and op2 entry (in row order, as the element makers enumerate them) the contribution
-// c_t c_l c_r x[a, b] is added when (a, b) is a superblock state (a and b in one sector) and
-// |c_t c_l c_r| > 1e-15, as the element makers drop it.
+// zc = coupling terms applied to x, the general form (KronDev::general).  A coupling term has
+// one operator on each half (op1 on LL or LR, op2 on RR or RL) and a sign that is a product of a
+// factor of the row's LLLR state and one of its RRRL state, so per term the builder lists,
+// for every LLLR state a', the states a it reaches with op1 and their coefficients (left parity
+// sign x op1 value), and likewise for every RRRL state b' (right parity sign x op2 value);
+// the term's own factor is its coefficient times the sign rule's constant.  One workgroup
+// per LLLR state a' of the output, its threads over the sector's RRRL states b': for each
+// term (in term order), op1 entry and op2 entry (in row order, as the element makers enumerate
+// them) the contribution c_t c_l c_r x[a, b] is added when (a, b) is a superblock state (a and
+// b in one sector) and |c_t c_l c_r| > 1e-15, as the element makers drop it.
 struct KronCross {
   int nt, na, nb;
   const double *ct;                         // per term
@@ -168,178 +167,111 @@ __global__ __launch_bounds__(256) void k_kron_cross(KronCross kc, const double *
   kron_cross_row(kc, blockIdx.x, x, z);
 }
 
-// One TM x TN tile of one of a sector's two dense products: the left one (M_L X, k over
-// the sector's LLLR states, written to zl) or the right one (X M_R^T, k over its RRRL
-// states, written to z).  k-slabs of kKt staged in LDS, double
-// buffered: the next slab's global loads are issued before the current slab's products
-// (kKt 16, or 32 for a longer product per slab behind the loads).
-// Outside the sector the operands are zero.  MFMA: the four wavefronts split the tile 2 x 2,
-// each computing its (TM/2) x (TN/2) part as blocks of v_mfma_f64_16x16x4 (A fragment: lane
-// l holds A[l % 16][l / 16]; B fragment: B[l / 16][l % 16]; result register v of lane l:
-// D[4 v + l / 16][l % 16], as a one-hot scan of the instruction on gfx950 shows).  Without
-// (64 x 64 only): each thread a 4 x 4 block of FP64 fused multiply-adds (rows ty + 16 i,
-// columns tx + 16 j).
-typedef double kron_v4d __attribute__((ext_vector_type(4)));
-
-template <int TM, int TN, bool MFMA, int kKt>
-__device__ __forceinline__ void kron_tile_body(const KronSector *sec, const int32_t *tiles, int32_t nt,
-                                               const double *__restrict__ ML, const double *__restrict__ MR,
-                                               const double *__restrict__ x, double *__restrict__ z,
-                                               double *__restrict__ zl, int xcd) {
-  static_assert(MFMA || (TM == 64 && TN == 64), "the vector form computes 64 x 64 tiles");
-  constexpr int PA = kKt * TM / 256, PB = kKt * TN / 256;   // staged elements per thread
-  constexpr int BM = TM / 32, BN = TN / 32;                 // 16 x 16 blocks per wavefront
-  __shared__ double As[2][kKt][TM + 1];   // As[buffer][k][row]
-  __shared__ double Bs[2][kKt][TN + 1];   // Bs[buffer][k][col]
-  // xcd: consecutive tiles (one sector's, in list order) to the blocks of one XCD, so that
-  // a sector's operands are fetched into one XCD's L2
-  const int32_t lt = xcd ? xcd_logical(blockIdx.x, nt) : (int32_t)blockIdx.x;
-  const int32_t *tl = tiles + 4 * (int64_t)lt;
-  const KronSector S = sec[tl[0]];
-  const int32_t r0 = tl[1] * TM, c0 = tl[2] * TN;
-  const bool right = tl[3] != 0;
-  const int32_t K = right ? S.db : S.da;
-  const double *X = x + S.off;
-  const double *Aop = right ? X : ML + S.ml;           // A[i][k] = Aop[(r0 + i) lda + k]
-  const int64_t lda = right ? S.db : S.da;
-  const double *Bop = right ? MR + S.mr : X;           // left: B[k][j] = X[k db + c0 + j]
-  double ra[PA], rb[PB];                               // right: B[k][j] = M_R[(c0 + j) db + k]
-  // staging geometry, fixed over the k loop: A element u of this thread is row
-  // tid / kKt + (256 / kKt) u of the tile at column tid % kKt of the slab (right B the same
-  // with rows of M_R); left B element u is k-row tid / TN + (256 / TN) u at column tid % TN
-  const int kA = threadIdx.x % kKt, iA = threadIdx.x / kKt;
-  const double *pA = Aop + (int64_t)(r0 + iA) * lda + kA;
-  const int64_t sA = (int64_t)(256 / kKt) * lda;
-  const int kB = right ? kA : threadIdx.x / TN;
-  const int jB = right ? iA : threadIdx.x % TN;
-  const double *pB = right ? Bop + (int64_t)(c0 + jB) * S.db + kA : Bop + (int64_t)kB * S.db + c0 + jB;
-  const int64_t sB = right ? (int64_t)(256 / kKt) * S.db : (int64_t)(256 / TN) * S.db;
-  auto fetch = [&](int32_t k0) {
-#pragma unroll
-    for (int u = 0; u < PA; u++) {
-      const bool ok = r0 + iA + (256 / kKt) * u < S.da && k0 + kA < K;
-      ra[u] = ok ? pA[u * sA + k0] : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < PB; u++) {
-      if (right) {
-        const bool ok = c0 + jB + (256 / kKt) * u < S.db && k0 + kA < K;
-        rb[u] = ok ? pB[u * sB + k0] : 0.0;
-      } else {
-        const bool ok = c0 + jB < S.db && k0 + kB + (256 / TN) * u < K;
-        rb[u] = ok ? pB[u * sB + (int64_t)k0 * S.db] : 0.0;
-      }
-    }
-  };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int u = 0; u < PA; u++) {
-      const int e = threadIdx.x + 256 * u;
-      As[buf][e % kKt][e / kKt] = ra[u];
-    }
-#pragma unroll
-    for (int u = 0; u < PB; u++) {
-      const int e = threadIdx.x + 256 * u;
-      if (right) Bs[buf][e % kKt][e / kKt] = rb[u];
-      else Bs[buf][e / TN][e % TN] = rb[u];
-    }
-  };
-  const int wave = threadIdx.x / 64, l = threadIdx.x % 64;
-  const int wr = (wave / 2) * (TM / 2), wc = (wave % 2) * (TN / 2);   // MFMA: this wavefront's part
-  const int li = l % 16, lk = l / 16;
-  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-  kron_v4d macc[BM][BN];
-  double vacc[4][4];
-#pragma unroll
-  for (int i = 0; i < BM; i++)
-#pragma unroll
-    for (int j = 0; j < BN; j++) macc[i][j] = kron_v4d{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) vacc[i][j] = 0.0;
-  fetch(0);
-  stage(0);
-  __syncthreads();
-  int buf = 0;
-  for (int32_t k0 = 0; k0 < K; k0 += kKt) {
-    const bool more = k0 + kKt < K;
-    if (more) fetch(k0 + kKt);
-    if constexpr (MFMA) {
-#pragma unroll
-      for (int kk = 0; kk < kKt; kk += 4) {
-        double a[BM], b[BN];
-#pragma unroll
-        for (int i = 0; i < BM; i++) a[i] = As[buf][kk + lk][wr + 16 * i + li];
-#pragma unroll
-        for (int j = 0; j < BN; j++) b[j] = Bs[buf][kk + lk][wc + 16 * j + li];
-#pragma unroll
-        for (int i = 0; i < BM; i++)
-#pragma unroll
-          for (int j = 0; j < BN; j++) macc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], macc[i][j], 0, 0, 0);
-      }
-    } else {
-#pragma unroll 2
-      for (int k = 0; k < kKt; k++) {
-        double av[4], bv[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) av[i] = As[buf][k][ty + 16 * i];
-#pragma unroll
-        for (int j = 0; j < 4; j++) bv[j] = Bs[buf][k][tx + 16 * j];
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-          for (int j = 0; j < 4; j++) vacc[i][j] = fma(av[i], bv[j], vacc[i][j]);
-      }
-    }
-    if (more) stage(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
-  }
-  double *Z = right ? z + S.off : zl + S.off;
-  auto put = [&](int32_t rr, int32_t cc, double v) {
-    if (rr < S.da && cc < S.db) {
-      const int64_t at = (int64_t)rr * S.db + cc;
-      Z[at] = v;
-    }
-  };
-  if constexpr (MFMA) {
-#pragma unroll
-    for (int bi = 0; bi < BM; bi++)
-#pragma unroll
-      for (int bj = 0; bj < BN; bj++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) put(r0 + wr + 16 * bi + 4 * v + lk, c0 + wc + 16 * bj + li, macc[bi][bj][v]);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) put(r0 + ty + 16 * i, c0 + tx + 16 * j, vacc[i][j]);
-  }
-}
-
-#define KRON_LAUNCH_ARGS                                                                     \
-  const KronSector *sec, const int32_t *tiles, int32_t nt, const double *ML, const double *MR, \
-      const double *x, double *z, double *zl, int xcd
-
-template <int TM, int TN, bool MFMA, int kKt = 16>
-__global__ __launch_bounds__(256) void k_kron_tile(KRON_LAUNCH_ARGS) {
-  kron_tile_body<TM, TN, MFMA, kKt>(sec, tiles, nt, ML, MR, x, z, zl, xcd);
-}
-// the 64 x 64 matrix-core tile held to at most 128 registers per lane, four wavefronts per
-// SIMD
-__global__ __launch_bounds__(256, 4) void k_kron_tile_o4(KRON_LAUNCH_ARGS) {
-  kron_tile_body<64, 64, true, 16>(sec, tiles, nt, ML, MR, x, z, zl, xcd);
-}
-
-// the 128 x 128 matrix-core tile held to two wavefronts per SIMD (at most 256 registers per
-// lane): half the operand traffic per output of the 64 x 64 tile
-__global__ __launch_bounds__(256, 2) void k_kron_tile_o2(KRON_LAUNCH_ARGS) {
-  kron_tile_body<128, 128, true, 16>(sec, tiles, nt, ML, MR, x, z, zl, xcd);
-}
-
 __global__ __launch_bounds__(256) void k_zero(int64_t n, double *p) {
   for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) p[i] = 0.0;
+}
+
+// Output tiles of t x t over all sectors, in launch order: the sectors cut into bands of whole
+// tile rows, the bands dealt to the eight XCDs (workgroup i runs on XCD i mod 8) by their work, so
+// that a band's operands are read into one L2 (KLM m = 799: L2 misses 1.8 M lines a product
+// against 4.0 M with the tiles dealt by length alone, a solve 83 ms against 92); each XCD's
+// bands longest k extent (da + db) first, so that the short tiles fill in behind the long ones.
+std::vector<KronTile> kron_tiles(const std::vector<KronSector> &sec, int32_t t) {
+  auto rows = [&](size_t s) { return (sec[s].da + t - 1) / t; };
+  auto cols = [&](size_t s) { return (sec[s].db + t - 1) / t; };
+  auto length = [&](size_t s) { return sec[s].da + sec[s].db; };
+  double total = 0.0;
+  for (size_t s = 0; s < sec.size(); s++) total += (double)rows(s) * cols(s) * length(s);
+  struct Band {
+    size_t sector;
+    int32_t i0, i1;
+    double work;
+  };
+  std::vector<Band> bands;
+  for (size_t s = 0; s < sec.size(); s++) {
+    const double row = (double)cols(s) * length(s);
+    const int32_t n = rows(s), cut = std::min(n, (int32_t)std::ceil(row * n / (total / (4 * kXcds))));
+    for (int32_t c = 0; c < cut; c++) {
+      const int32_t i0 = (int32_t)((int64_t)n * c / cut), i1 = (int32_t)((int64_t)n * (c + 1) / cut);
+      bands.push_back(Band{s, i0, i1, row * (i1 - i0)});
+    }
+  }
+  std::stable_sort(bands.begin(), bands.end(), [](const Band &a, const Band &b) { return a.work > b.work; });
+  double load[kXcds] = {};
+  std::vector<Band> mine[kXcds];
+  for (const Band &b : bands) {
+    const int q = (int)(std::min_element(load, load + kXcds) - load);
+    load[q] += b.work;
+    mine[q].push_back(b);
+  }
+  std::vector<KronTile> queue[kXcds], out;
+  for (int q = 0; q < kXcds; q++) {
+    std::stable_sort(mine[q].begin(), mine[q].end(),
+                     [&](const Band &a, const Band &b) { return length(a.sector) > length(b.sector); });
+    for (const Band &b : mine[q])
+      for (int32_t i = b.i0; i < b.i1; i++)
+        for (int32_t j = 0; j < cols(b.sector); j++) queue[q].emplace_back(sec[b.sector], i * t, j * t);
+  }
+  size_t nt = 0, at[kXcds] = {};
+  for (const auto &q : queue) nt += q.size();
+  for (size_t p = 0; p < nt; p++) {
+    int q = (int)(p % kXcds);
+    if (at[q] == queue[q].size())   // used up: the one with most left
+      for (int k = 0; k < kXcds; k++)
+        if (queue[k].size() - at[k] > queue[q].size() - at[q]) q = k;
+    out.push_back(queue[q][at[q]++]);
+  }
+  return out;
+}
+
+// 32 x 32 tiles once there are enough of them to keep the 256 CUs' four slots each busy
+// through a good part of the launch; below, 16 x 16 tiles, whose chains are shorter and which
+// are four times as many.  Solves, microseconds a step, 16 x 16 against 32 x 32: Hubbard m = 396
+// (208 tiles of 32) 18.9 and 20.4, KLM m = 280 (313) 23.6 and 23.6, m = 400 (580) 41.1 and 35.5,
+// m = 799 (2133) 196 and 107.
+int kron_shape_rule(const KronDev &K) { return K.ntiles[1] >= 400 ? 1 : 0; }
+
+// The short form of the coupling terms (KronMap) from their lists; false if some term has a
+// state with several targets, or with targets in several sectors.
+bool kron_maps(const KronDev &K, const std::vector<int32_t> &asec, const std::vector<int32_t> &bsec,
+               const std::vector<double> &ct, const std::vector<int32_t> &lptr, const std::vector<int32_t> &lidx,
+               const std::vector<double> &lval, const std::vector<int32_t> &rptr, const std::vector<int32_t> &ridx,
+               const std::vector<double> &rval, std::vector<KronMap> &lmap, std::vector<KronMap> &rmap) {
+  const int nt = (int)ct.size();
+  lmap.assign((size_t)nt * K.na, KronMap{0.0, -1, 0});
+  rmap.assign((size_t)nt * K.nb, KronMap{0.0, -1, 0});
+  for (int t = 0; t < nt; t++) {
+    const int32_t *lp = lptr.data() + (size_t)t * (K.na + 1), *rp = rptr.data() + (size_t)t * (K.nb + 1);
+    for (const KronSector &S : K.hsec) {
+      int32_t sa = -1, sb = -1;   // target sectors
+      for (int32_t i = S.a0; i < S.a0 + S.da; i++) {
+        if (lp[i + 1] - lp[i] > 1) return false;
+        for (int32_t e = lp[i]; e < lp[i + 1]; e++) {
+          const int32_t q = asec[lidx[e]];
+          if (sa >= 0 && q != sa) return false;
+          sa = q;
+        }
+      }
+      for (int32_t i = S.b0; i < S.b0 + S.db; i++) {
+        if (rp[i + 1] - rp[i] > 1) return false;
+        for (int32_t e = rp[i]; e < rp[i + 1]; e++) {
+          const int32_t q = bsec[ridx[e]];
+          if (sb >= 0 && q != sb) return false;
+          sb = q;
+        }
+      }
+      if (sa < 0 || sa != sb) continue;
+      const KronSector &T = K.hsec[sa];
+      for (int32_t i = S.a0; i < S.a0 + S.da; i++)
+        if (lp[i + 1] > lp[i]) {
+          const int32_t e = lp[i];
+          lmap[(size_t)t * K.na + i] = KronMap{ct[t] * lval[e], (int32_t)(T.off + (int64_t)(lidx[e] - T.a0) * T.db), 0};
+        }
+      for (int32_t i = S.b0; i < S.b0 + S.db; i++)
+        if (rp[i + 1] > rp[i]) rmap[(size_t)t * K.nb + i] = KronMap{rval[rp[i]], ridx[rp[i]] - T.b0, 0};
+    }
+  }
+  return true;
 }
 
 bool left_kind(int k) { return k == K_LL || k == K_LR || k == K_LLLR; }
@@ -347,52 +279,13 @@ bool right_kind(int k) { return k == K_RR || k == K_RL || k == K_RRRL; }
 
 }  // namespace
 
-// The coupling terms (to zc) on a side stream, beside the dense tiles (to z and zl) on the
-// caller's stream: the tiles are queued first and hold four workgroups per CU, the coupling
-// terms' workgroups, which need no LDS, fill the room beside them.
-void KronDev::product(const double *x, hipStream_t s) const {
+int KronDev::shape() const { return variant == 0 ? 0 : variant == 2 ? 1 : rule; }
+
+void KronDev::cross(const double *x, hipStream_t s) const {
+  if (!general || na == 0) return;
   const KronCross kc{ncross, na, nb, ct.p, lptr.p, lidx.p, rptr.p, ridx.p, lval.p, rval.p, asec.p, bsec.p, sec.p};
-  const int shape = kKronShape[variant];
-  const int nt = ntiles[shape];
-  if (!side) {
-    HIPCHK(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
-    HIPCHK(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&join, hipEventDisableTiming));
-  }
-  if (na > 0) HIPCHK(hipEventRecord(fork, s));   // x is ready, and the last product's zc has been read
-  if (nt > 0) {
-    const int32_t *tl = tiles[shape].p;
-    // live timing (dmrgx_profile_begin_sampled): HIP events around the dense products, their
-    // floating-point operations counted where the CRS products count bytes
-    Context &C = ctx();
-    std::pair<hipEvent_t, hipEvent_t> *ev = nullptr;
-    if (C.prof_take()) {
-      ev = C.prof_slot();
-      HIPCHK(hipEventRecord(ev->first, s));
-      C.prof_bytes += flops;
-    }
-#define KRON_ARGS sec.p, tl, nt, ML.p, MR.p, x, z.p, zl.p, xcd
-    switch (variant) {
-      case 0: k_kron_tile<64, 64, false><<<nt, 256, 0, s>>>(KRON_ARGS); break;
-      case 1: k_kron_tile<64, 64, true><<<nt, 256, 0, s>>>(KRON_ARGS); break;
-      case 2: k_kron_tile<128, 128, true><<<nt, 256, 0, s>>>(KRON_ARGS); break;
-      case 3: k_kron_tile<64, 128, true><<<nt, 256, 0, s>>>(KRON_ARGS); break;
-      case 4: k_kron_tile<128, 64, true><<<nt, 256, 0, s>>>(KRON_ARGS); break;
-      case 5: k_kron_tile<64, 64, true, 32><<<nt, 256, 0, s>>>(KRON_ARGS); break;
-      case 6: k_kron_tile_o4<<<nt, 256, 0, s>>>(KRON_ARGS); break;
-      default: k_kron_tile_o2<<<nt, 256, 0, s>>>(KRON_ARGS); break;
-    }
-#undef KRON_ARGS
-    if (ev) HIPCHK(hipEventRecord(ev->second, s));
-    HIPCHK(hipGetLastError());
-  }
-  if (na > 0) {
-    HIPCHK(hipStreamWaitEvent(side, fork, 0));
-    k_kron_cross<<<na, 256, 0, side>>>(kc, x, zc.p);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipEventRecord(join, side));
-    HIPCHK(hipStreamWaitEvent(s, join, 0));   // zc complete before the epilogue
-  }
+  k_kron_cross<<<na, 256, 0, s>>>(kc, x, zc.p);
+  HIPCHK(hipGetLastError());
 }
 
 }  // namespace dmrgx
@@ -480,34 +373,20 @@ int dmrgx_superblock_kron(const dmrgx_superblock *S, dmrgx_kron **out) {
     K.na = (int32_t)aLL.size();
     K.nb = (int32_t)bRR.size();
     int64_t ml = 0, mr = 0;
-    std::vector<int32_t> tiles[kKronShapes];
-    for (int s = 0; s < K.nsec; s++) {
-      KronSector &sc = K.hsec[s];
+    for (KronSector &sc : K.hsec) {
+      const int64_t na16 = (sc.da + 15) / 16, nb16 = (sc.db + 15) / 16;
       sc.ml = ml;
       sc.mr = mr;
-      ml += (int64_t)sc.da * sc.da;
-      mr += (int64_t)sc.db * sc.db;
+      ml += na16 * na16 * 256;
+      mr += nb16 * nb16 * 256;
       K.flops += 2.0 * sc.da * sc.db * (double)(sc.da + sc.db);
-      for (int sh = 0; sh < kKronShapes; sh++)
-        for (int ph = 0; ph < 2; ph++)   // the left and the right product of each tile
-          for (int32_t ti = 0; ti * kKronTM[sh] < sc.da; ti++)
-            for (int32_t tj = 0; tj * kKronTN[sh] < sc.db; tj++) {
-              tiles[sh].push_back(s);
-              tiles[sh].push_back(ti);
-              tiles[sh].push_back(tj);
-              tiles[sh].push_back(ph);
-            }
     }
-    // longest first (k extent of the tile's product: da for the left, db for the right one),
-    // so that the short tiles fill in behind the long ones instead of the long ones ending last
+    std::vector<KronTile> tiles[kKronShapes];
     for (int sh = 0; sh < kKronShapes; sh++) {
-      std::vector<std::array<int32_t, 4>> t(tiles[sh].size() / 4);
-      std::memcpy(t.data(), tiles[sh].data(), sizeof(int32_t) * tiles[sh].size());
-      auto klen = [&](const std::array<int32_t, 4> &a) { return a[3] ? K.hsec[a[0]].db : K.hsec[a[0]].da; };
-      std::stable_sort(t.begin(), t.end(), [&](const auto &a, const auto &b) { return klen(a) > klen(b); });
-      std::memcpy(tiles[sh].data(), t.data(), sizeof(int32_t) * tiles[sh].size());
-      K.ntiles[sh] = (int32_t)t.size();
+      tiles[sh] = kron_tiles(K.hsec, kKronTile[sh]);
+      K.ntiles[sh] = (int32_t)tiles[sh].size();
     }
+    K.rule = kron_shape_rule(K);
     // the term list split by the halves it acts on
     std::vector<int32_t> left, right, cross;
     for (size_t i = 0; i < S->hterms.size(); i++) {
@@ -561,9 +440,6 @@ int dmrgx_superblock_kron(const dmrgx_superblock *S, dmrgx_kron **out) {
           }
         };
         ct.push_back((t.sign_mode == 1 ? -1.0 : 1.0) * t.coeff);
-        const int32_t base_l = (int32_t)lidx.size(), base_r = (int32_t)ridx.size();
-        (void)base_l;
-        (void)base_r;
         for (int32_t i = 0; i < K.na; i++) {
           lptr.push_back((int32_t)lidx.size());
           const int q[2] = {aLL[i], aLR[i]};
@@ -600,13 +476,24 @@ int dmrgx_superblock_kron(const dmrgx_superblock *S, dmrgx_kron **out) {
         buf.resize(std::max<size_t>(h.size(), 1));
         if (!h.empty()) ctx().copy_in(buf.p, h.data(), sizeof(T) * h.size());
       };
-      upl(K.ct, ct);
-      upl(K.lptr, lptr);
-      upl(K.lidx, lidx);
-      upl(K.lval, lval);
-      upl(K.rptr, rptr);
-      upl(K.ridx, ridx);
-      upl(K.rval, rval);
+      // the short form: at most one target per state and term, and per term and sector one
+      // target sector on each half (an operator of a site changes the quantum numbers by a
+      // fixed amount); a term and sector whose target sectors differ contributes nothing
+      std::vector<KronMap> lmap, rmap;
+      K.general = !kron_maps(K, asec, bsec, ct, lptr, lidx, lval, rptr, ridx, rval, lmap, rmap);
+      if (K.general) {
+        upl(K.ct, ct);
+        upl(K.lptr, lptr);
+        upl(K.lidx, lidx);
+        upl(K.lval, lval);
+        upl(K.rptr, rptr);
+        upl(K.ridx, ridx);
+        upl(K.rval, rval);
+        K.zc.resize(n);
+      } else {
+        upl(K.lmap, lmap);
+        upl(K.rmap, rmap);
+      }
     }
     auto up = [](auto &buf, const auto &h) {
       using T = typename std::decay_t<decltype(h)>::value_type;
@@ -615,7 +502,6 @@ int dmrgx_superblock_kron(const dmrgx_superblock *S, dmrgx_kron **out) {
     };
     up(K.sec, K.hsec);
     for (int sh = 0; sh < kKronShapes; sh++) up(K.tiles[sh], tiles[sh]);
-    up(K.cross, cross);
     DevBuf<int16_t> daLL, daLR, dbRR, dbRL;
     DevBuf<int32_t> dleft, dright;
     up(daLL, aLL);
@@ -640,9 +526,6 @@ int dmrgx_superblock_kron(const dmrgx_superblock *S, dmrgx_kron **out) {
       k_kron_right<<<(K.nb + 255) / 256, 256, 0, st>>>(kb, S->terms.p, dright.p, (int)right.size(), S->ops.p,
                                                        S->ele_ptrs.p, K.MR.p);
     HIPCHK(hipGetLastError());
-    K.z.resize(std::max<int32_t>(n, 1));
-    K.zl.resize(std::max<int32_t>(n, 1));
-    K.zc.resize(std::max<int32_t>(n, 1));
     HIPCHK(hipStreamSynchronize(st));   // the build's own buffers go out of scope
     *out = H.release();
   });
@@ -658,9 +541,8 @@ int dmrgx_kron_info(const dmrgx_kron *K, int32_t *n, int32_t *sectors, int32_t *
 }
 
 int dmrgx_kron_set_kernel(dmrgx_kron *K, int32_t variant) {
-  if (!K || variant < 0 || variant >= 2 * kKronVariants) return DMRGX_ERR_ARG;
-  K->K.variant = variant % kKronVariants;
-  K->K.xcd = variant / kKronVariants;
+  if (!K || variant < 0 || variant >= kKronVariants) return DMRGX_ERR_ARG;
+  K->K.variant = variant;
   return DMRGX_OK;
 }
 
@@ -669,44 +551,38 @@ int dmrgx_kron_autotune(dmrgx_kron *K, int32_t *variant_out, double *us_out) {
   return run_status([&] {
     KronDev &D = K->K;
     hipStream_t st = ctx().stream;
-    DevBuf<double> x(std::max<int32_t>(D.n, 1));
+    DevBuf<double> x(std::max<int32_t>(D.n, 1)), y(std::max<int32_t>(D.n, 1));
     launch_start_vector(D.n, 7, x.p, st);
     hipEvent_t e0, e1;
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
-    int best = D.variant, best_xcd = D.xcd;
+    int best = kKronDefault;
     float best_ms = 1e30f, dflt_ms = 1e30f;
-    for (int c = 0; c < 2 * kKronVariants; c++) {
-      const int v = c % kKronVariants, xm = c / kKronVariants;
+    for (int v : {kKronDefault, 0, 2}) {
       D.variant = v;
-      D.xcd = xm;
-      D.product(x.p, st);
+      launch_spmv(op_of(D), x.p, y.p, st);
       HIPCHK(hipEventRecord(e0, st));
-      for (int r = 0; r < 5; r++) D.product(x.p, st);
+      for (int r = 0; r < 5; r++) launch_spmv(op_of(D), x.p, y.p, st);
       HIPCHK(hipEventRecord(e1, st));
       HIPCHK(hipEventSynchronize(e1));
       float ms = 0;
       HIPCHK(hipEventElapsedTime(&ms, e0, e1));
-      if (c == kKronDefault) dflt_ms = ms;
+      if (v == kKronDefault) dflt_ms = ms;
       if (ms < best_ms) {
         best_ms = ms;
         best = v;
-        best_xcd = xm;
       }
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    // the default kernel stays unless another is more than 2 % faster: the five products'
-    // timing varies by about 1 %, and between the two 64 x 64 kernels, which time within
-    // that, whole solves favour the default-occupancy one
+    // the default stays unless another is more than 2 % faster: the five products' timing
+    // varies by about 1 %
     if (dflt_ms <= 1.02f * best_ms) {
       best_ms = dflt_ms;
-      best = kKronDefault % kKronVariants;
-      best_xcd = kKronDefault / kKronVariants;
+      best = kKronDefault;
     }
     D.variant = best;
-    D.xcd = best_xcd;
-    if (variant_out) *variant_out = best + kKronVariants * best_xcd;
+    if (variant_out) *variant_out = best;
     if (us_out) *us_out = best_ms * 1000.0 / 5;
   });
 }
@@ -715,14 +591,10 @@ int dmrgx_kron_spmv(const dmrgx_kron *K, const double *x, double *y) {
   if (!K || !x || !y) return DMRGX_ERR_ARG;
   return run_status([&] {
     const int32_t n = K->K.n;
-    DevBuf<double> dx(n);
+    DevBuf<double> dx(n), dy(n);
     ctx().copy_in(dx.p, x, sizeof(double) * n);
-    K->K.product(dx.p, ctx().stream);
-    std::vector<double> zl(n), zc(n);
-    ctx().copy_out(y, K->K.z.p, sizeof(double) * n);
-    ctx().copy_out(zl.data(), K->K.zl.p, sizeof(double) * n);
-    ctx().copy_out(zc.data(), K->K.zc.p, sizeof(double) * n);
-    for (int32_t i = 0; i < n; i++) y[i] = (y[i] + zl[i]) + zc[i];   // as the solvers' epilogue sums them
+    launch_spmv(op_of(K->K), dx.p, dy.p, ctx().stream);
+    ctx().copy_out(y, dy.p, sizeof(double) * n);
   });
 }
 

@@ -135,3 +135,80 @@ def test_gpu_residual_stop(path):
         K.free()
         A.free()
         sb.free()
+
+
+def _random_superblock(left, right, middle, seed, far=False):
+    """A spin-1/2 superblock with left[i] / right[i] block states of 2 S^z = left0 + 2 i, random
+    block operators of the right selection rules, and the terms of an XXZ chain; with far also
+    couplings of block to block and of block to site, whose operators take a state to many."""
+    from dmrg_c_amd import snapshot as S
+    rng = np.random.default_rng(seed)
+    qa = np.repeat(np.arange(len(left)), left) * 2 - (len(left) - 1)
+    qb = np.repeat(np.arange(len(right)), right) * 2 - (len(right) - 1)
+    site = np.array([1, -1])
+
+    def op(q, dq, sym=False):
+        a = np.where(q[:, None] == q[None, :] + dq, rng.uniform(-1, 1, (len(q), len(q))), 0.0)
+        return a + a.T if sym else a
+
+    def crs(a):
+        r, c = np.nonzero(a)
+        row = np.zeros(len(a) + 1, np.int64)
+        np.add.at(row, r + 1, 1)
+        return S.Crs(len(a), len(a), np.cumsum(row), c.astype(np.int32), a[r, c])
+    sp = np.array([[0.0, 1.0], [0.0, 0.0]])
+    sz = np.diag([0.5, -0.5])
+    pa, pb = op(qa, 2), op(qb, 2)
+    mats = [op(qa, 0, True), op(qb, 0, True), sz, sp, sp.T, pa, pa.T, pb, pb.T]
+    rows = [("LL", 0, -1, 1.0), ("RR", 1, -1, 0.7), ("LR", 2, -1, 0.3), ("RL", 2, -1, -0.2),
+            ("LLLR", 5, 4, 0.5), ("LLLR", 6, 3, 0.5), ("RRRL", 7, 4, 0.4), ("RRRL", 8, 3, 0.4)]
+    if middle:
+        rows += [("LRRL", 3, 4, 0.5), ("LRRL", 4, 3, 0.5), ("LRRL", 2, 2, 1.1)]
+    if far:
+        rows += [("LLRR", 5, 8, 0.25), ("LLRR", 6, 7, 0.25), ("LLRL", 5, 4, 0.1), ("LLRL", 6, 3, 0.1),
+                 ("LRRR", 3, 8, 0.2), ("LRRR", 4, 7, 0.2)]
+    rows += [("ZERO", -1, -1, 0.0)]
+    terms = np.zeros(len(rows), S.TERM_DTYPE)
+    for t, (kind, o1, o2, c) in zip(terms, rows):
+        t["kind"], t["op1"], t["op2"], t["coeff"] = S.KIND_NAMES.index(kind), o1, o2, c
+        t["ele0"] = t["ele1"] = t["ele2"] = -1
+    sa, sb = (qa[:, None] + site).ravel(), (qb[:, None] + site).ravel()
+    states = [(x, y) for s in np.unique(sa) for x in np.nonzero(sa == s)[0] for y in np.nonzero(sb == -s)[0]]
+    x, y = np.array(states).T
+    basis = [np.ascontiguousarray(v, np.int16) for v in (x // 2, x % 2, y // 2, y % 2)]
+    return S.Snapshot(len(x), len(qa), len(qb), 2, 0, 0, 0, *basis, [crs(m) for m in mats], [], terms)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("variant", [0, 1, 2], ids=["16x16", "by-size", "32x32"])
+@pytest.mark.parametrize("left,right,far", [([1], [1], False), ([1, 1], [1, 1], False), ([1, 14, 2], [2, 13, 1], False),
+                                            ([8, 9, 8], [7, 9, 8], True), ([1, 15, 16, 17], [33, 1, 15, 30], False),
+                                            ([10, 34, 5], [3, 36, 17], True)],
+                         ids=["1", "2", "edge16", "far17", "edge32", "far"])
+def test_gpu_kron_tile_edges(left, right, far, variant):
+    """Sectors of one state, of one below, at and one above 16 and 32 states on either side (the
+    shifted last slab, partly filled tiles), and couplings in their general form, against the
+    product with the oracle's CRS."""
+    import dmrg_c_amd as D
+    import oracle_py as O
+    import scipy.sparse as sp
+    s = _random_superblock(left, right, True, 7, far)
+    row, col, val = O.assemble(s)
+    A = sp.csr_matrix((val, col, row), shape=(s.n, s.n))
+    A = (A + A.T - sp.diags(A.diagonal())).tocsr()
+    sb = D.Superblock(s)
+    K = sb.kron()
+    K.set_kernel(variant)
+    try:
+        x = np.random.default_rng(3).standard_normal(s.n)
+        y, y_ref = K.matvec(x), A @ x
+        # each element sums at most a few hundred products of numbers below 2
+        assert np.abs(y - y_ref).max() <= 1e-13 * np.abs(x).max() * abs(A).sum(axis=1).max()
+        if s.n < 3000:
+            E, _, _ = K.ground_state()
+            w = np.linalg.eigvalsh(A.toarray())
+            assert abs(E - w[0]) <= 1e-10 * max(1.0, abs(w[0]))
+    finally:
+        K.free()
+        sb.free()
+
