@@ -251,7 +251,8 @@ struct ArrOp {
 };
 
 int64_t build_basis_device(const dmrgx_basis_qn &q, DevBuf<int16_t> &LL, DevBuf<int16_t> &LR, DevBuf<int16_t> &RR,
-                           DevBuf<int16_t> &RL);
+                           DevBuf<int16_t> &RL, std::vector<BasisSector> &sec, std::vector<int16_t> &a_half,
+                           std::vector<int16_t> &b_half);
 
 // The basis comes from the caller's arrays (LL..RL, host) or, with qn set, is built on the
 // device from the blocks' quantum numbers (n, dim_LL, dim_RR, d are then taken from qn).
@@ -265,7 +266,7 @@ static dmrgx_superblock *create_superblock(int32_t n, int32_t dim_LL, int32_t di
     dim_LL = qn->dim_LL;
     dim_RR = qn->dim_RR;
     d = qn->dim_onsite;
-    n = (int32_t)build_basis_device(*qn, S->LL, S->LR, S->RR, S->RL);
+    n = (int32_t)build_basis_device(*qn, S->LL, S->LR, S->RR, S->RL, S->qn_sec, S->qn_a, S->qn_b);
   }
   if (n <= 0 || dim_LL <= 0 || dim_RR <= 0 || d <= 0) throw Failure(DMRGX_ERR_ARG, "superblock dimensions must be positive");
   if ((int)terms_in.size() > kMaxTerms) throw Failure(DMRGX_ERR_ARG, "too many terms");
@@ -330,16 +331,15 @@ static dmrgx_superblock *create_superblock(int32_t n, int32_t dim_LL, int32_t di
   S->hele.resize(eles.size());
   for (size_t i = 0; i < eles.size(); i++) S->hele[i].assign(eles[i].first, eles[i].first + eles[i].second);
   hipStream_t st = ctx().stream;
-  auto up16 = [&](DevBuf<int16_t> &b, const int16_t *h) {
-    b.resize(n);
-    ctx().copy_in(b.p, h, sizeof(int16_t) * n);
-  };
   if (!qn) {
-    up16(S->LL, LL);
-    up16(S->LR, LR);
-    up16(S->RR, RR);
-    up16(S->RL, RL);
+    for (DevBuf<int16_t> *b : {&S->LL, &S->LR, &S->RR, &S->RL}) b->resize(n);
+    ctx().copy_in_many({{S->LL.p, LL, sizeof(int16_t) * n},
+                        {S->LR.p, LR, sizeof(int16_t) * n},
+                        {S->RR.p, RR, sizeof(int16_t) * n},
+                        {S->RL.p, RL, sizeof(int16_t) * n}});
   }
+  // operators, parity arrays, terms and the tables of their device addresses in one transfer
+  Upload up;
   std::vector<DOp> hops(std::max<size_t>(ops.size(), 1));
   S->op_row.resize(ops.size());
   S->op_col.resize(ops.size());
@@ -347,30 +347,32 @@ static dmrgx_superblock *create_superblock(int32_t n, int32_t dim_LL, int32_t di
   for (size_t i = 0; i < ops.size(); i++) {
     const ArrOp &a = ops[i];
     const int64_t nnz = a.row[a.row_dim];
-    S->op_row[i].resize((size_t)a.row_dim + 1);
-    S->op_col[i].resize(std::max<int64_t>(nnz, 1));
-    S->op_val[i].resize(std::max<int64_t>(nnz, 1));
-    ctx().copy_in(S->op_row[i].p, a.row, sizeof(int64_t) * ((size_t)a.row_dim + 1));
-    if (nnz) {
-      ctx().copy_in(S->op_col[i].p, a.col, sizeof(int32_t) * nnz);
-      ctx().copy_in(S->op_val[i].p, a.val, sizeof(double) * nnz);
-    }
-    hops[i] = DOp{S->op_row[i].p, S->op_col[i].p, S->op_val[i].p};
+    up.add(S->op_row[i], a.row, (size_t)a.row_dim + 1);
+    up.add(S->op_col[i], a.col, (size_t)nnz);
+    up.add(S->op_val[i], a.val, (size_t)nnz);
   }
   std::vector<const int32_t *> heles(std::max<size_t>(eles.size(), 1), nullptr);
   S->ele.resize(eles.size());
-  for (size_t i = 0; i < eles.size(); i++) {
-    S->ele[i].resize(std::max(eles[i].second, 1));
-    ctx().copy_in(S->ele[i].p, eles[i].first, sizeof(int32_t) * eles[i].second);
-    heles[i] = S->ele[i].p;
+  for (size_t i = 0; i < eles.size(); i++) up.add(S->ele[i], eles[i].first, (size_t)eles[i].second);
+  up.add(S->ops, hops);
+  up.add(S->terms, terms);
+  up.add(S->ele_ptrs, heles);
+  up.place(S->pack);
+  for (size_t i = 0; i < ops.size(); i++) hops[i] = DOp{S->op_row[i].p, S->op_col[i].p, S->op_val[i].p};
+  for (size_t i = 0; i < eles.size(); i++) heles[i] = S->ele[i].p;
+  up.send();
+  S->hop.resize(ops.size());
+  for (const DTerm &t : terms) {
+    if (t.kind < K_LLRL || t.kind > K_LRRR) continue;   // the kinds that couple the halves
+    for (int o : {t.op1, t.op2}) {
+      const ArrOp &a = ops[o];
+      if (!S->hop[o].row.empty()) continue;
+      const int64_t nnz = a.row[a.row_dim];
+      S->hop[o].row.assign(a.row, a.row + a.row_dim + 1);
+      S->hop[o].col.assign(a.col, a.col + nnz);
+      S->hop[o].val.assign(a.val, a.val + nnz);
+    }
   }
-  S->ops.resize(hops.size());
-  ctx().copy_in(S->ops.p, hops.data(), sizeof(DOp) * hops.size());
-  S->terms.resize(std::max<size_t>(terms.size(), 1));
-  if (!terms.empty())
-    ctx().copy_in(S->terms.p, terms.data(), sizeof(DTerm) * terms.size());
-  S->ele_ptrs.resize(heles.size());
-  ctx().copy_in(S->ele_ptrs.p, heles.data(), sizeof(const int32_t *) * heles.size());
   // dense superblock inverse, -1 where absent (GET_BASIS_SUPERBLOCK.c Inv fill)
   const int64_t dim_whole = (int64_t)dim_LL * d * dim_RR * d;
   if (dim_whole > (int64_t)1 << 34) throw Failure(DMRGX_ERR_ARG, "superblock product space too large for the dense inverse");
@@ -378,8 +380,7 @@ static dmrgx_superblock *create_superblock(int32_t n, int32_t dim_LL, int32_t di
   k_fill_int<<<1024, 256, 0, st>>>(dim_whole, -1, S->inv.p);
   k_inv_scatter<<<(n + 255) / 256, 256, 0, st>>>(S->view(), S->inv.p);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(st));  // host arrays above go out of scope
-  return S.release();
+  return S.release();   // no wait: the host arrays have been read, users of the device ones queue behind
 }
 
 void fill_inverse(int32_t n, int32_t dim_RR, int32_t d, const int16_t *LL, const int16_t *LR, const int16_t *RR,

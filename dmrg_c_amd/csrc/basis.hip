@@ -22,16 +22,10 @@
 #include <utility>
 #include <vector>
 
-#include "entry.h"
+#include "superblock.h"
 
 namespace dmrgx {
 namespace {
-
-struct BasisSector {
-  int64_t off;       // first superblock row of the sector
-  int32_t dB;        // right states per left state
-  int32_t a0, b0;    // first left / right state of the sector in the packed lists
-};
 
 // One thread per superblock row: binary search of its sector, then the left state of the
 // row (row / dB within the sector) and the right state (row % dB).
@@ -106,19 +100,23 @@ int64_t basis_sectors(const dmrgx_basis_qn &q, std::vector<BasisSector> &sec, st
   return n;
 }
 
-// Device basis arrays of the sector (LL, LR, RR, RL resized to n); returns n.
+// Device basis arrays of the sector (LL, LR, RR, RL resized to n) and the host lists they
+// come from; returns n.
 int64_t build_basis_device(const dmrgx_basis_qn &q, DevBuf<int16_t> &LL, DevBuf<int16_t> &LR, DevBuf<int16_t> &RR,
-                           DevBuf<int16_t> &RL) {
-  std::vector<BasisSector> sec;
-  std::vector<int16_t> a_half, b_half;
+                           DevBuf<int16_t> &RL, std::vector<BasisSector> &sec, std::vector<int16_t> &a_half,
+                           std::vector<int16_t> &b_half) {
   const int64_t n = basis_sectors(q, sec, a_half, b_half);
   if (n == 0) throw Failure(DMRGX_ERR_ARG, "no state of the blocks reaches the target quantum numbers");
   Context &C = ctx();
-  DevBuf<BasisSector> dsec(sec.size());
-  DevBuf<int16_t> da(a_half.size()), db(b_half.size());
-  C.copy_in(dsec.p, sec.data(), sizeof(BasisSector) * sec.size());
-  C.copy_in(da.p, a_half.data(), sizeof(int16_t) * a_half.size());
-  C.copy_in(db.p, b_half.data(), sizeof(int16_t) * b_half.size());
+  DevBuf<char> mem;
+  DevView<BasisSector> dsec;
+  DevView<int16_t> da, db;
+  Upload up;
+  up.add(dsec, sec);
+  up.add(da, a_half);
+  up.add(db, b_half);
+  up.place(mem);
+  up.send();
   LL.resize(n);
   LR.resize(n);
   RR.resize(n);
@@ -145,7 +143,9 @@ int dmrgx_superblock_basis(const dmrgx_basis_qn *q, int64_t *n_out, int16_t *LL,
       return;
     }
     DevBuf<int16_t> dLL, dLR, dRR, dRL;
-    const int64_t n = build_basis_device(*q, dLL, dLR, dRR, dRL);
+    std::vector<BasisSector> sec;
+    std::vector<int16_t> a_half, b_half;
+    const int64_t n = build_basis_device(*q, dLL, dLR, dRR, dRL, sec, a_half, b_half);
     Context &C = ctx();
     C.copy_out(LL, dLL.p, sizeof(int16_t) * n);
     C.copy_out(LR, dLR.p, sizeof(int16_t) * n);

@@ -196,6 +196,35 @@ void Context::copy_in_many(const std::vector<CopySeg> &segs) {
   if (chunks > 1) HIPCHK(hipEventSynchronize(xfer_ev[chunks & 1]));
 }
 
+void Upload::send() const {
+  Context &C = ctx();
+  xfer_init(C);
+  // the buffer's bytes kXferChunk at a time through the pinned chunks
+  const size_t chunks = (total + kXferChunk - 1) / kXferChunk;
+  size_t it = 0;   // first item that reaches into the chunk
+  for (size_t k = 0; k < chunks; k++) {
+    const size_t lo = k * kXferChunk, hi = std::min(total, lo + kXferChunk);
+    if (k >= 2) HIPCHK(hipEventSynchronize(C.xfer_ev[k & 1]));   // chunk k - 2's DMA has read the buffer
+    while (it < items.size() && items[it].off + items[it].bytes <= lo) it++;
+    for (size_t i = it; i < items.size() && items[i].off < hi; i++) {
+      const size_t a = std::max(lo, items[i].off), b = std::min(hi, items[i].off + items[i].bytes);
+      if (a < b)
+        std::memcpy(C.xfer_pin[k & 1] + (a - lo), static_cast<const char *>(items[i].src) + (a - items[i].off), b - a);
+    }
+    HIPCHK(hipMemcpyAsync(base + lo, C.xfer_pin[k & 1], hi - lo, hipMemcpyHostToDevice, C.stream));
+    HIPCHK(hipEventRecord(C.xfer_ev[k & 1], C.stream));
+  }
+  if (chunks > 0) HIPCHK(hipEventSynchronize(C.xfer_ev[(chunks - 1) & 1]));
+  if (chunks > 1) HIPCHK(hipEventSynchronize(C.xfer_ev[chunks & 1]));
+}
+
+std::vector<char> Upload::block() const {
+  std::vector<char> b(total);
+  for (const Item &i : items)
+    if (i.bytes) std::memcpy(b.data() + i.off, i.src, i.bytes);
+  return b;
+}
+
 hipEvent_t *Context::step_events() {
   if (!step_ev[0])
     for (int i = 0; i < 2; i++) HIPCHK(hipEventCreateWithFlags(&step_ev[i], hipEventDisableTiming));

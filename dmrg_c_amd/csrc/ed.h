@@ -6,25 +6,27 @@
 struct dmrgx_ed {
   int32_t L = 0, d = 0;
   int64_t n = 0;
-  dmrgx::DevBuf<int64_t> basis, pw;
+  dmrgx::DevBuf<int64_t> basis;
+  dmrgx::DevBuf<char> pack;      // what the views below point into
+  dmrgx::DevView<int64_t> pw;
   std::vector<std::vector<int64_t>> hrow;
   std::vector<std::vector<int32_t>> hcol;
   std::vector<std::vector<double>> hval;
-  std::vector<dmrgx::DevBuf<int64_t>> op_row;
-  std::vector<dmrgx::DevBuf<int32_t>> op_col;
-  std::vector<dmrgx::DevBuf<double>> op_val;
+  std::vector<dmrgx::DevView<int64_t>> op_row;
+  std::vector<dmrgx::DevView<int32_t>> op_col;
+  std::vector<dmrgx::DevView<double>> op_val;
   std::vector<dmrgx_ed_term> hterms;
   std::vector<int32_t> hn_ele;
-  std::vector<int64_t> hpw;     // host sources of the uploads, kept until the problem is freed
-  std::vector<char> hops;
-  dmrgx::DevBuf<dmrgx_ed_term> terms;
-  dmrgx::DevBuf<int32_t> n_ele;
+  std::vector<int64_t> hpw;
+  std::vector<char> hpack;      // host source of the upload, kept until the problem is freed
+  dmrgx::DevView<dmrgx_ed_term> terms;
+  dmrgx::DevView<int32_t> n_ele;
   struct DOp {
     const int64_t *row;
     const int32_t *col;
     const double *val;
   };
-  dmrgx::DevBuf<DOp> ops;
+  dmrgx::DevView<DOp> ops;
 };
 
 namespace dmrgx {

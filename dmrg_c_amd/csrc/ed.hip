@@ -300,34 +300,27 @@ std::unique_ptr<dmrgx_ed> ed_setup(int32_t L, int32_t d, int32_t n_ops, const CR
   std::vector<int64_t> &pw = E->hpw;
   pw.assign(L + 1, 1);
   for (int s = 1; s <= L; s++) pw[s] = pw[s - 1] * d;
-  E->pw.resize(L + 1);
-  HIPCHK(hipMemcpyAsync(E->pw.p, pw.data(), sizeof(int64_t) * (L + 1), hipMemcpyHostToDevice, st));
+  // operators, terms and tables in one buffer and one queued copy
+  Upload up;
   std::vector<DOp> hops(std::max(n_ops, 1));
   E->op_row.resize(n_ops);
   E->op_col.resize(n_ops);
   E->op_val.resize(n_ops);
+  up.add(E->pw, pw);
   for (int32_t i = 0; i < n_ops; i++) {
-    const size_t nnz = E->hcol[i].size();
-    E->op_row[i].resize(d + 1);
-    E->op_col[i].resize(std::max<size_t>(nnz, 1));
-    E->op_val[i].resize(std::max<size_t>(nnz, 1));
-    HIPCHK(hipMemcpyAsync(E->op_row[i].p, E->hrow[i].data(), sizeof(int64_t) * (d + 1), hipMemcpyHostToDevice, st));
-    if (nnz) {
-      HIPCHK(hipMemcpyAsync(E->op_col[i].p, E->hcol[i].data(), sizeof(int32_t) * nnz, hipMemcpyHostToDevice, st));
-      HIPCHK(hipMemcpyAsync(E->op_val[i].p, E->hval[i].data(), sizeof(double) * nnz, hipMemcpyHostToDevice, st));
-    }
-    hops[i] = DOp{E->op_row[i].p, E->op_col[i].p, E->op_val[i].p};
+    up.add(E->op_row[i], E->hrow[i]);
+    up.add(E->op_col[i], E->hcol[i]);
+    up.add(E->op_val[i], E->hval[i]);
   }
-  E->ops.resize(hops.size());
-  E->hops.assign(reinterpret_cast<const char *>(hops.data()), reinterpret_cast<const char *>(hops.data() + hops.size()));
-  HIPCHK(hipMemcpyAsync(E->ops.p, E->hops.data(), sizeof(DOp) * hops.size(), hipMemcpyHostToDevice, st));
-  E->terms.resize(std::max<size_t>(E->hterms.size(), 1));
-  if (!E->hterms.empty())
-    HIPCHK(hipMemcpyAsync(E->terms.p, E->hterms.data(), sizeof(dmrgx_ed_term) * E->hterms.size(),
-                          hipMemcpyHostToDevice, st));
-  E->n_ele.resize(d);
-  if (n_ele) HIPCHK(hipMemcpyAsync(E->n_ele.p, E->hn_ele.data(), sizeof(int32_t) * d, hipMemcpyHostToDevice, st));
-  // no wait: the host arrays copied from live in E until it is freed, and every user of the
+  static_assert(sizeof(DOp) == sizeof(dmrgx_ed::DOp), "same layout");
+  up.add(E->ops, reinterpret_cast<const dmrgx_ed::DOp *>(hops.data()), hops.size());
+  up.add(E->terms, E->hterms);
+  up.add(E->n_ele, E->hn_ele.data(), E->hn_ele.size());
+  up.place(E->pack);
+  for (int32_t i = 0; i < n_ops; i++) hops[i] = DOp{E->op_row[i].p, E->op_col[i].p, E->op_val[i].p};
+  E->hpack = up.block();
+  HIPCHK(hipMemcpyAsync(E->pack.p, E->hpack.data(), E->hpack.size(), hipMemcpyHostToDevice, st));
+  // no wait: the host block copied from lives in E until it is freed, and every user of the
   // device copies is queued behind the copies on this stream
   return E;
 }

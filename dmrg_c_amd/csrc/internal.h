@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <limits>
 #include <cstdio>
@@ -120,6 +121,48 @@ struct DevBuf {
     p = nullptr;
     count = 0;
   }
+};
+
+// A device array inside a buffer that something else owns.
+template <class T>
+struct DevView {
+  T *p = nullptr;
+  size_t count = 0;
+};
+
+// Several host arrays brought to the device in one buffer and one transfer: every
+// synchronised copy of its own costs ~15 us, which is what a call with a few dozen small
+// operators and tables used to wait for.  add() each array, place() sets the views (device
+// addresses that other arrays hold can be taken now), send() copies.  The host arrays live until
+// send() returns, and their contents are read there.
+class Upload {
+ public:
+  template <class T>
+  void add(DevView<T> &v, const T *src, size_t n) {
+    items.push_back(Item{src, n * sizeof(T), total, reinterpret_cast<void **>(&v.p)});
+    v.count = n;
+    total += (std::max<size_t>(n * sizeof(T), 1) + 255) / 256 * 256;
+  }
+  template <class T>
+  void add(DevView<T> &v, const std::vector<T> &src) { add(v, src.data(), src.size()); }
+  void place(DevBuf<char> &mem) {
+    mem.resize(total);
+    base = mem.p;
+    for (const Item &i : items) *i.view = base + i.off;
+  }
+  void send() const;
+  // the bytes of the buffer as one host block, for a copy that the caller queues itself
+  std::vector<char> block() const;
+  char *base = nullptr;
+  size_t total = 0;
+
+ private:
+  struct Item {
+    const void *src;
+    size_t bytes, off;
+    void **view;
+  };
+  std::vector<Item> items;
 };
 
 }  // namespace dmrgx
@@ -818,11 +861,13 @@ struct EdRows {
 // sub-Hamiltonians, obc.cpp).
 struct ObcDev {
   int32_t n = 0, dim_LL = 0, dim_RR = 0, d = 0, lanes = 8;
-  DevBuf<int16_t> LL, LR, RR, RL, LL_LLLR, LR_LLLR, LR_LRRL, RL_LRRL, RR_RRRL, RL_RRRL;
-  DevBuf<int32_t> inv, inv_LLLR, inv_LRRL, inv_RRRL, ele_RR;
-  DevBuf<int64_t> r1, r2, r3, r4;
-  DevBuf<int32_t> c1, c2, c3, c4;
-  DevBuf<double> v1, v2, v3, v4;
+  DevBuf<char> pack;   // what the views point into
+  DevView<int16_t> LL, LR, RR, RL, LL_LLLR, LR_LLLR, LR_LRRL, RL_LRRL, RR_RRRL, RL_RRRL;
+  DevView<int32_t> inv_LLLR, inv_LRRL, inv_RRRL, ele_RR;
+  DevBuf<int32_t> inv;
+  DevView<int64_t> r1, r2, r3, r4;
+  DevView<int32_t> c1, c2, c3, c4;
+  DevView<double> v1, v2, v3, v4;
   ObcRows rows() const {
     return ObcRows{dim_RR, d, LL.p, LR.p, RR.p, RL.p, inv.p, inv_LLLR.p, inv_LRRL.p, inv_RRRL.p,
                    LL_LLLR.p, LR_LLLR.p, LR_LRRL.p, RL_LRRL.p, RR_RRRL.p, RL_RRRL.p,
@@ -915,19 +960,20 @@ struct KronDev {
   int rule = 0;                           // the shape that kKronDefault takes
   const dmrgx_superblock *sb = nullptr;   // borrowed: basis, inverse, operators, term list
   std::vector<KronSector> hsec;
-  DevBuf<KronSector> sec;
+  DevBuf<char> pack;                      // what the views below point into
+  DevView<KronSector> sec;
   DevBuf<double> ML, MR;                  // dense sector blocks (kron_at)
-  DevBuf<KronTile> tiles[kKronShapes];
-  DevBuf<KronMap> lmap, rmap;             // per coupling term and state
+  DevView<KronTile> tiles[kKronShapes];
+  DevView<KronMap> lmap, rmap;            // per coupling term and state
   // The general form of the coupling terms, kept when some state has more than one target
   // under a term (operators of a block, not of a site): per term its factor, and the LLLR / RRRL
   // states each state reaches with the term's operator on that half (k_kron_cross, into zc
   // before the product kernel).
   bool general = false;
-  DevBuf<double> ct, lval, rval;
-  DevBuf<int32_t> lptr, lidx, rptr, ridx;
+  DevView<double> ct, lval, rval;
+  DevView<int32_t> lptr, lidx, rptr, ridx;
   // flat LLLR / RRRL state of (LL d + LR) / (RR d + RL) (-1: none) and each flat state's sector
-  DevBuf<int32_t> aidx, bidx, asec, bsec;
+  DevView<int32_t> aidx, bidx, asec, bsec;
   DevBuf<double> zc;
   double flops = 0.0;                     // of the two dense products per H x
   int shape() const;

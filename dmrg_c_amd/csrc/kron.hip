@@ -312,51 +312,76 @@ int dmrgx_superblock_kron(const dmrgx_superblock *S, dmrgx_kron **out) {
     K.n = n;
     K.sb = S;
     hipStream_t st = ctx().stream;
-    // the basis (host copy) and its sectors
-    std::vector<int16_t> LL(n), LR(n), RR(n), RL(n);
-    ctx().copy_out(LL.data(), S->LL.p, sizeof(int16_t) * n);
-    ctx().copy_out(LR.data(), S->LR.p, sizeof(int16_t) * n);
-    ctx().copy_out(RR.data(), S->RR.p, sizeof(int16_t) * n);
-    ctx().copy_out(RL.data(), S->RL.p, sizeof(int16_t) * n);
     std::vector<int16_t> aLL, aLR, bRR, bRL;
     std::vector<int32_t> asec, bsec;
-    int64_t r = 0;
-    while (r < n) {
-      KronSector sc{};
-      sc.off = r;
-      // db: rows until (LL, LR) changes; da: runs of db rows with the same RRRL sequence
-      int64_t e = r;
-      while (e < n && LL[e] == LL[r] && LR[e] == LR[r]) e++;
-      sc.db = (int32_t)(e - r);
-      int64_t a = r;
-      while (a < n && a + sc.db <= n && RR[a] == RR[r] && RL[a] == RL[r]) a += sc.db;
-      sc.da = (int32_t)((a - r) / sc.db);
-      // every row of the sector must be (LLLR state i, RRRL state j) at off + i db + j
-      // the product check: every row run of the sector has one (LL, LR) and the first run's
-      // RRRL sequence
-      for (int32_t i = 0; i < sc.da; i++) {
-        const int64_t q0 = r + (int64_t)i * sc.db;
-        int same = std::memcmp(&RR[q0], &RR[r], sizeof(int16_t) * sc.db) == 0 &&
-                   std::memcmp(&RL[q0], &RL[r], sizeof(int16_t) * sc.db) == 0;
-        const int16_t ll = LL[q0], lr = LR[q0];
-        for (int32_t j = 1; j < sc.db; j++) same &= (int)(LL[q0 + j] == ll) & (int)(LR[q0 + j] == lr);
-        if (!same) throw Failure(DMRGX_ERR_ARG, "superblock basis is not a product of LLLR and RRRL states per sector");
+    if (!S->qn_sec.empty()) {
+      // the sectors as the basis was built from them
+      for (size_t s = 0; s < S->qn_sec.size(); s++) {
+        const BasisSector &q = S->qn_sec[s];
+        const bool end = s + 1 == S->qn_sec.size();
+        KronSector sc{};
+        sc.off = q.off;
+        sc.db = q.dB;
+        sc.da = (end ? (int32_t)(S->qn_a.size() / 2) : S->qn_sec[s + 1].a0) - q.a0;
+        sc.a0 = (int32_t)aLL.size();
+        sc.b0 = (int32_t)bRR.size();
+        for (int32_t i = 0; i < sc.da; i++) {
+          aLL.push_back(S->qn_a[2 * (q.a0 + i)]);
+          aLR.push_back(S->qn_a[2 * (q.a0 + i) + 1]);
+          asec.push_back(K.nsec);
+        }
+        for (int32_t j = 0; j < sc.db; j++) {
+          bRR.push_back(S->qn_b[2 * (q.b0 + j)]);
+          bRL.push_back(S->qn_b[2 * (q.b0 + j) + 1]);
+          bsec.push_back(K.nsec);
+        }
+        K.hsec.push_back(sc);
+        K.nsec++;
       }
-      sc.a0 = (int32_t)aLL.size();
-      sc.b0 = (int32_t)bRR.size();
-      for (int32_t i = 0; i < sc.da; i++) {
-        aLL.push_back(LL[r + (int64_t)i * sc.db]);
-        aLR.push_back(LR[r + (int64_t)i * sc.db]);
-        asec.push_back(K.nsec);
+    } else {   // the basis (host copy) and its sectors
+      std::vector<int16_t> LL(n), LR(n), RR(n), RL(n);
+      ctx().copy_out(LL.data(), S->LL.p, sizeof(int16_t) * n);
+      ctx().copy_out(LR.data(), S->LR.p, sizeof(int16_t) * n);
+      ctx().copy_out(RR.data(), S->RR.p, sizeof(int16_t) * n);
+      ctx().copy_out(RL.data(), S->RL.p, sizeof(int16_t) * n);
+      int64_t r = 0;
+      while (r < n) {
+        KronSector sc{};
+        sc.off = r;
+        // db: rows until (LL, LR) changes; da: runs of db rows with the same RRRL sequence
+        int64_t e = r;
+        while (e < n && LL[e] == LL[r] && LR[e] == LR[r]) e++;
+        sc.db = (int32_t)(e - r);
+        int64_t a = r;
+        while (a < n && a + sc.db <= n && RR[a] == RR[r] && RL[a] == RL[r]) a += sc.db;
+        sc.da = (int32_t)((a - r) / sc.db);
+        // every row of the sector must be (LLLR state i, RRRL state j) at off + i db + j
+        // the product check: every row run of the sector has one (LL, LR) and the first run's
+        // RRRL sequence
+        for (int32_t i = 0; i < sc.da; i++) {
+          const int64_t q0 = r + (int64_t)i * sc.db;
+          int same = std::memcmp(&RR[q0], &RR[r], sizeof(int16_t) * sc.db) == 0 &&
+                     std::memcmp(&RL[q0], &RL[r], sizeof(int16_t) * sc.db) == 0;
+          const int16_t ll = LL[q0], lr = LR[q0];
+          for (int32_t j = 1; j < sc.db; j++) same &= (int)(LL[q0 + j] == ll) & (int)(LR[q0 + j] == lr);
+          if (!same) throw Failure(DMRGX_ERR_ARG, "superblock basis is not a product of LLLR and RRRL states per sector");
+        }
+        sc.a0 = (int32_t)aLL.size();
+        sc.b0 = (int32_t)bRR.size();
+        for (int32_t i = 0; i < sc.da; i++) {
+          aLL.push_back(LL[r + (int64_t)i * sc.db]);
+          aLR.push_back(LR[r + (int64_t)i * sc.db]);
+          asec.push_back(K.nsec);
+        }
+        for (int32_t j = 0; j < sc.db; j++) {
+          bRR.push_back(RR[r + j]);
+          bRL.push_back(RL[r + j]);
+          bsec.push_back(K.nsec);
+        }
+        K.hsec.push_back(sc);
+        K.nsec++;
+        r += (int64_t)sc.da * sc.db;
       }
-      for (int32_t j = 0; j < sc.db; j++) {
-        bRR.push_back(RR[r + j]);
-        bRL.push_back(RL[r + j]);
-        bsec.push_back(K.nsec);
-      }
-      K.hsec.push_back(sc);
-      K.nsec++;
-      r += (int64_t)sc.da * sc.db;
     }
     // state -> flat index maps (each LLLR / RRRL state belongs to one sector)
     std::vector<int32_t> aidx((size_t)S->dim_LL * d, -1), bidx((size_t)S->dim_RR * d, -1);
@@ -397,28 +422,16 @@ int dmrgx_superblock_kron(const dmrgx_superblock *S, dmrgx_kron **out) {
     }
     K.ncross = (int32_t)cross.size();
     // the coupling terms' per-state lists (see k_kron_cross), from host copies of the operators
+    std::vector<double> ct, lval, rval;
+    std::vector<int32_t> lptr, lidx, rptr, ridx;
+    std::vector<KronMap> lmap, rmap;
+    Upload up;
     {
-      auto op_host = [&](int id, std::vector<int64_t> &r, std::vector<int32_t> &c, std::vector<double> &v) {
-        r.resize(S->op_row[id].count);
-        ctx().copy_out(r.data(), S->op_row[id].p, sizeof(int64_t) * r.size());
-        const int64_t nnz = r.back();
-        c.resize(std::max<int64_t>(nnz, 1));
-        v.resize(std::max<int64_t>(nnz, 1));
-        if (nnz > 0) {
-          ctx().copy_out(c.data(), S->op_col[id].p, sizeof(int32_t) * nnz);
-          ctx().copy_out(v.data(), S->op_val[id].p, sizeof(double) * nnz);
-        }
-      };
-      std::vector<double> ct;
-      std::vector<int32_t> lptr, lidx, rptr, ridx;
-      std::vector<double> lval, rval;
       for (int32_t ci : cross) {
         const DTerm &t = S->hterms[ci];
-        std::vector<int64_t> r1, r2;
-        std::vector<int32_t> c1, c2;
-        std::vector<double> v1, v2;
-        op_host(t.op1, r1, c1, v1);
-        op_host(t.op2, r2, c2, v2);
+        const auto &r1 = S->hop[t.op1].row, &r2 = S->hop[t.op2].row;
+        const auto &c1 = S->hop[t.op1].col, &c2 = S->hop[t.op2].col;
+        const auto &v1 = S->hop[t.op1].val, &v2 = S->hop[t.op2].val;
         auto par = [&](int e, int state) { return S->hele[e][state]; };
         // parity of the row's LLLR part and of its RRRL part in the term's sign rule
         auto left_parity = [&](int ll, int lr) {
@@ -471,49 +484,40 @@ int dmrgx_superblock_kron(const dmrgx_superblock *S, dmrgx_kron **out) {
       }
       if ((int64_t)lidx.size() > INT32_MAX / 2 || (int64_t)ridx.size() > INT32_MAX / 2)
         throw Failure(DMRGX_ERR_ARG, "coupling-term lists too long");
-      auto upl = [](auto &buf, const auto &h) {
-        using T = typename std::decay_t<decltype(h)>::value_type;
-        buf.resize(std::max<size_t>(h.size(), 1));
-        if (!h.empty()) ctx().copy_in(buf.p, h.data(), sizeof(T) * h.size());
-      };
       // the short form: at most one target per state and term, and per term and sector one
       // target sector on each half (an operator of a site changes the quantum numbers by a
       // fixed amount); a term and sector whose target sectors differ contributes nothing
-      std::vector<KronMap> lmap, rmap;
       K.general = !kron_maps(K, asec, bsec, ct, lptr, lidx, lval, rptr, ridx, rval, lmap, rmap);
       if (K.general) {
-        upl(K.ct, ct);
-        upl(K.lptr, lptr);
-        upl(K.lidx, lidx);
-        upl(K.lval, lval);
-        upl(K.rptr, rptr);
-        upl(K.ridx, ridx);
-        upl(K.rval, rval);
+        up.add(K.ct, ct);
+        up.add(K.lptr, lptr);
+        up.add(K.lidx, lidx);
+        up.add(K.lval, lval);
+        up.add(K.rptr, rptr);
+        up.add(K.ridx, ridx);
+        up.add(K.rval, rval);
         K.zc.resize(n);
       } else {
-        upl(K.lmap, lmap);
-        upl(K.rmap, rmap);
+        up.add(K.lmap, lmap);
+        up.add(K.rmap, rmap);
       }
     }
-    auto up = [](auto &buf, const auto &h) {
-      using T = typename std::decay_t<decltype(h)>::value_type;
-      buf.resize(std::max<size_t>(h.size(), 1));
-      if (!h.empty()) ctx().copy_in(buf.p, h.data(), sizeof(T) * h.size());
-    };
-    up(K.sec, K.hsec);
-    for (int sh = 0; sh < kKronShapes; sh++) up(K.tiles[sh], tiles[sh]);
-    DevBuf<int16_t> daLL, daLR, dbRR, dbRL;
-    DevBuf<int32_t> dleft, dright;
-    up(daLL, aLL);
-    up(daLR, aLR);
-    up(dbRR, bRR);
-    up(dbRL, bRL);
-    up(K.asec, asec);
-    up(K.bsec, bsec);
-    up(K.aidx, aidx);
-    up(K.bidx, bidx);
-    up(dleft, left);
-    up(dright, right);
+    up.add(K.sec, K.hsec);
+    for (int sh = 0; sh < kKronShapes; sh++) up.add(K.tiles[sh], tiles[sh]);
+    DevView<int16_t> daLL, daLR, dbRR, dbRL;   // read by the kernels below only
+    DevView<int32_t> dleft, dright;
+    up.add(daLL, aLL);
+    up.add(daLR, aLR);
+    up.add(dbRR, bRR);
+    up.add(dbRL, bRL);
+    up.add(K.asec, asec);
+    up.add(K.bsec, bsec);
+    up.add(K.aidx, aidx);
+    up.add(K.bidx, bidx);
+    up.add(dleft, left);
+    up.add(dright, right);
+    up.place(K.pack);
+    up.send();
     K.ML.resize(std::max<int64_t>(ml, 1));
     K.MR.resize(std::max<int64_t>(mr, 1));
     k_zero<<<1024, 256, 0, st>>>(ml, K.ML.p);
@@ -526,8 +530,7 @@ int dmrgx_superblock_kron(const dmrgx_superblock *S, dmrgx_kron **out) {
       k_kron_right<<<(K.nb + 255) / 256, 256, 0, st>>>(kb, S->terms.p, dright.p, (int)right.size(), S->ops.p,
                                                        S->ele_ptrs.p, K.MR.p);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(st));   // the build's own buffers go out of scope
-    *out = H.release();
+    *out = H.release();   // no wait: the host lists have been read, products queue behind the build
   });
 }
 

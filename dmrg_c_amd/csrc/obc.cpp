@@ -20,22 +20,16 @@ using namespace dmrgx;
 
 namespace {
 
-template <class T>
-void up(DevBuf<T> &b, const T *h, size_t n) {
-  b.resize(n ? n : 1);
-  if (n) ctx().copy_in(b.p, h, sizeof(T) * n);
-}
-
-void up_crs(const CRS1 *M, int rows_needed, int col_limit, DevBuf<int64_t> &r, DevBuf<int32_t> &c,
-            DevBuf<double> &v, const char *name) {
+void up_crs(Upload &u, const CRS1 *M, int rows_needed, int col_limit, DevView<int64_t> &r, DevView<int32_t> &c,
+            DevView<double> &v, const char *name) {
   if (M->row_dim < rows_needed) throw Failure(DMRGX_ERR_ARG, std::string(name) + " has fewer rows than its sub-basis");
   const int64_t nnz = M->Row[rows_needed];
   for (int64_t j = 0; j < nnz; j++)
     if (M->Col[j] < 0 || M->Col[j] >= col_limit)
       throw Failure(DMRGX_ERR_ARG, std::string(name) + " has a column outside its sub-basis");
-  up(r, reinterpret_cast<const int64_t *>(M->Row), (size_t)rows_needed + 1);
-  up(c, M->Col, nnz);
-  up(v, M->Val, nnz);
+  u.add(r, reinterpret_cast<const int64_t *>(M->Row), (size_t)rows_needed + 1);
+  u.add(c, M->Col, (size_t)nnz);
+  u.add(v, M->Val, (size_t)nnz);
 }
 
 std::unique_ptr<ObcDev> upload_obc(const CRS1 *M_LLLR, const CRS1 *M_LRRL, const CRS1 *M_LRRL_Sign,
@@ -74,26 +68,27 @@ std::unique_ptr<ObcDev> upload_obc(const CRS1 *M_LLLR, const CRS1 *M_LRRL, const
   for (int i = 0; i < B->dim_RRRL; i++)
     if (B->RR_RRRL[i] < 0 || B->RR_RRRL[i] >= dr || B->RL_RRRL[i] < 0 || B->RL_RRRL[i] >= d)
       throw Failure(DMRGX_ERR_ARG, "RRRL sub-basis outside its blocks");
-  up(O->LL, B->LL_LLLRRRRL, n);
-  up(O->LR, B->LR_LLLRRRRL, n);
-  up(O->RR, B->RR_LLLRRRRL, n);
-  up(O->RL, B->RL_LLLRRRRL, n);
-  up(O->inv_LLLR, iLLLR.data(), iLLLR.size());
-  up(O->inv_LRRL, iLRRL.data(), iLRRL.size());
-  up(O->inv_RRRL, iRRRL.data(), iRRRL.size());
-  up(O->LL_LLLR, B->LL_LLLR, B->dim_LLLR);
-  up(O->LR_LLLR, B->LR_LLLR, B->dim_LLLR);
-  up(O->LR_LRRL, B->LR_LRRL, B->dim_LRRL);
-  up(O->RL_LRRL, B->RL_LRRL, B->dim_LRRL);
-  up(O->RR_RRRL, B->RR_RRRL, B->dim_RRRL);
-  up(O->RL_RRRL, B->RL_RRRL, B->dim_RRRL);
-  up_crs(M_LLLR, B->dim_LLLR, B->dim_LLLR, O->r1, O->c1, O->v1, "M_LLLR");
-  up_crs(M_LRRL, B->dim_LRRL, B->dim_LRRL, O->r2, O->c2, O->v2, "M_LRRL");
+  Upload u;
+  u.add(O->LL, B->LL_LLLRRRRL, n);
+  u.add(O->LR, B->LR_LLLRRRRL, n);
+  u.add(O->RR, B->RR_LLLRRRRL, n);
+  u.add(O->RL, B->RL_LLLRRRRL, n);
+  u.add(O->inv_LLLR, iLLLR);
+  u.add(O->inv_LRRL, iLRRL);
+  u.add(O->inv_RRRL, iRRRL);
+  u.add(O->LL_LLLR, B->LL_LLLR, B->dim_LLLR);
+  u.add(O->LR_LLLR, B->LR_LLLR, B->dim_LLLR);
+  u.add(O->LR_LRRL, B->LR_LRRL, B->dim_LRRL);
+  u.add(O->RL_LRRL, B->RL_LRRL, B->dim_LRRL);
+  u.add(O->RR_RRRL, B->RR_RRRL, B->dim_RRRL);
+  u.add(O->RL_RRRL, B->RL_RRRL, B->dim_RRRL);
+  up_crs(u, M_LLLR, B->dim_LLLR, B->dim_LLLR, O->r1, O->c1, O->v1, "M_LLLR");
+  up_crs(u, M_LRRL, B->dim_LRRL, B->dim_LRRL, O->r2, O->c2, O->v2, "M_LRRL");
   // M_LRRL_Sign is indexed by the LRRL state; the reference passes an empty matrix
   // (xxz_vf DIAGONALIZE_SUPERBLOCK.c:18) sized dim_LLLR, so accept any row count >= what
   // its stored rows cover and treat missing rows as empty.
+  std::vector<int64_t> rows((size_t)B->dim_LRRL + 1, 0);
   {
-    std::vector<int64_t> rows((size_t)B->dim_LRRL + 1, 0);
     const int avail = std::min(M_LRRL_Sign->row_dim, B->dim_LRRL);
     for (int i = 0; i <= avail; i++) rows[i] = M_LRRL_Sign->Row[i];
     for (int i = avail + 1; i <= B->dim_LRRL; i++) rows[i] = rows[avail];
@@ -101,12 +96,14 @@ std::unique_ptr<ObcDev> upload_obc(const CRS1 *M_LLLR, const CRS1 *M_LRRL, const
     for (int64_t j = 0; j < nnz; j++)
       if (M_LRRL_Sign->Col[j] < 0 || M_LRRL_Sign->Col[j] >= B->dim_LRRL)
         throw Failure(DMRGX_ERR_ARG, "M_LRRL_Sign has a column outside its sub-basis");
-    up(O->r3, rows.data(), rows.size());
-    up(O->c3, M_LRRL_Sign->Col, nnz);
-    up(O->v3, M_LRRL_Sign->Val, nnz);
+    u.add(O->r3, rows);
+    u.add(O->c3, M_LRRL_Sign->Col, nnz);
+    u.add(O->v3, M_LRRL_Sign->Val, nnz);
   }
-  up_crs(M_RRRL, B->dim_RRRL, B->dim_RRRL, O->r4, O->c4, O->v4, "M_RRRL");
-  up(O->ele_RR, Ele_RR, (size_t)max_rr + 1);
+  up_crs(u, M_RRRL, B->dim_RRRL, B->dim_RRRL, O->r4, O->c4, O->v4, "M_RRRL");
+  u.add(O->ele_RR, Ele_RR, (size_t)max_rr + 1);
+  u.place(O->pack);
+  u.send();
   const int64_t dim_whole = (int64_t)dl * d * dr * d;
   O->inv.resize(dim_whole);
   fill_inverse(n, dr, d, O->LL.p, O->LR.p, O->RR.p, O->RL.p, O->inv.p, dim_whole, ctx().stream);
@@ -115,7 +112,6 @@ std::unique_ptr<ObcDev> upload_obc(const CRS1 *M_LLLR, const CRS1 *M_LRRL, const
   int g = 1;
   while (g < 64 && g * 3 < avg) g <<= 1;
   O->lanes = g;
-  HIPCHK(hipStreamSynchronize(ctx().stream));
   return O;
 }
 

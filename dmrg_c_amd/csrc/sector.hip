@@ -236,29 +236,23 @@ int dmrgx_v_m_sector(dmrgx_whole_basis *W, int32_t slot, const CRS1 *M, int32_t 
     if (S.n == 0) return;
     Context &C = ctx();
     hipStream_t st = C.stream;
-    DevBuf<int64_t> row(slot_dim + 1);
-    DevBuf<int32_t> col(nnz > 0 ? nnz : 1);
-    DevBuf<double> val(nnz > 0 ? nnz : 1), x(dim_in > 0 ? dim_in : 1), y(S.n);
-    C.copy_in(row.p, M->Row, sizeof(int64_t) * (slot_dim + 1));
-    if (nnz > 0) {
-      C.copy_in(col.p, M->Col, sizeof(int32_t) * nnz);
-      C.copy_in(val.p, M->Val, sizeof(double) * nnz);
-    }
-    if (dim_in > 0) C.copy_in(x.p, V, sizeof(double) * dim_in);
-    DevBuf<int32_t> eL, eLR, eR, bad(1);
-    if (sign) {
-      eL.resize(W->dim_LL);
-      C.copy_in(eL.p, ele_LL, sizeof(int32_t) * W->dim_LL);
-      if (slot >= 2) {
-        eLR.resize(W->d);
-        C.copy_in(eLR.p, ele_LR, sizeof(int32_t) * W->d);
-      }
-      if (slot >= 3) {
-        eR.resize(W->dim_RR);
-        C.copy_in(eR.p, ele_RR, sizeof(int32_t) * W->dim_RR);
-      }
-    }
-    HIPCHK(hipMemsetAsync(bad.p, 0, sizeof(int32_t), st));
+    DevBuf<char> mem;
+    DevView<int64_t> row;
+    DevView<int32_t> col, eL, eLR, eR, bad;
+    DevView<double> val, x;
+    const int32_t none = 0;
+    Upload up;
+    up.add(row, reinterpret_cast<const int64_t *>(M->Row), (size_t)slot_dim + 1);
+    up.add(col, M->Col, (size_t)nnz);
+    up.add(val, M->Val, (size_t)nnz);
+    up.add(bad, &none, 1);
+    if (sign) up.add(eL, ele_LL, (size_t)W->dim_LL);
+    if (sign && slot >= 2) up.add(eLR, ele_LR, (size_t)W->d);
+    if (sign && slot >= 3) up.add(eR, ele_RR, (size_t)W->dim_RR);
+    up.add(x, V, (size_t)std::max(dim_in, 0));
+    up.place(mem);
+    up.send();
+    DevBuf<double> y(S.n);
     k_v_m_sector<<<(unsigned)((S.n + 255) / 256), 256, 0, st>>>(
         S.n, slot, W->dim_RR, W->d, S.LL.p, S.LR.p, S.RR.p, S.RL.p, W->inv.p, row.p, col.p, val.p,
         sign ? eL.p : nullptr, eLR.p, eR.p, dim_in, x.p, y.p, bad.p);

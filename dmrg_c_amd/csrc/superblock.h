@@ -14,6 +14,12 @@ enum { ROLE_LL = 0, ROLE_RR = 1, ROLE_ON = 2 };
 inline constexpr int kSlot1[K_COUNT] = {S_LL, S_LR, S_RR, S_RL, S_LL, S_LL, S_LL, S_LR, S_LR, S_RR, -1};
 inline constexpr int kSlot2[K_COUNT] = {-1, -1, -1, -1, S_LR, S_RL, S_RR, S_RL, S_RR, S_RL, -1};
 
+struct BasisSector {
+  int64_t off;       // first superblock row of the sector
+  int32_t dB;        // right states per left state
+  int32_t a0, b0;    // first left / right state of the sector in the packed lists
+};
+
 constexpr double kZero = 1.0e-15;  // dmrg/DMRG_MAKE_ELEM_LL_LLLRRRRL.c:18
 constexpr int kMaxTerms = 256;
 
@@ -54,13 +60,24 @@ struct dmrgx_superblock {
   int32_t n = 0, dim_LL = 0, dim_RR = 0, d = 0, nt = 0, has_zero = 0;
   dmrgx::DevBuf<int16_t> LL, LR, RR, RL;
   dmrgx::DevBuf<int32_t> inv;
-  std::vector<dmrgx::DevBuf<int64_t>> op_row;
-  std::vector<dmrgx::DevBuf<int32_t>> op_col;
-  std::vector<dmrgx::DevBuf<double>> op_val;
-  std::vector<dmrgx::DevBuf<int32_t>> ele;
-  dmrgx::DevBuf<dmrgx::DOp> ops;
-  dmrgx::DevBuf<dmrgx::DTerm> terms;
-  dmrgx::DevBuf<const int32_t *> ele_ptrs;
+  dmrgx::DevBuf<char> pack;   // operators, parity arrays and terms: what the views point into
+  std::vector<dmrgx::DevView<int64_t>> op_row;
+  std::vector<dmrgx::DevView<int32_t>> op_col;
+  std::vector<dmrgx::DevView<double>> op_val;
+  std::vector<dmrgx::DevView<int32_t>> ele;
+  dmrgx::DevView<dmrgx::DOp> ops;
+  dmrgx::DevView<dmrgx::DTerm> terms;
+  dmrgx::DevView<const int32_t *> ele_ptrs;
+  // host copies of the operators of the coupling terms (for the Kronecker form's state lists)
+  struct HostOp {
+    std::vector<int64_t> row;
+    std::vector<int32_t> col;
+    std::vector<double> val;
+  };
+  std::vector<HostOp> hop;
+  // the basis' sectors and their left / right states, when it was built from quantum numbers
+  std::vector<dmrgx::BasisSector> qn_sec;
+  std::vector<int16_t> qn_a, qn_b;
   std::vector<dmrgx::DTerm> hterms;   // host copy of terms (without ZERO and zero-coefficient terms)
   std::vector<std::vector<int32_t>> hele;   // host copies of the parity arrays
   // last assembled lower triangle
