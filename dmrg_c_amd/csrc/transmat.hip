@@ -14,7 +14,7 @@
 // order, skipping the zeros of W: the same nonzero terms in the same order as the
 // reference's (the terms the reference adds for M1(i, r) = 0 are signed zeros, which do not
 // change a sum).  The file is built without FMA contraction, so Out is the reference's bit
-// for bit.  The dense result is compacted into the caller's CRS1 on the host.
+// for bit.  The dense result is compacted on the device.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -29,40 +29,55 @@ namespace {
 
 constexpr double kDropBelow = 1e-15;
 
-// dense[r][j] = M3(r, j) from CCS (col_ptr over columns, row indices per entry)
-__global__ __launch_bounds__(256) void k_ccs_to_dense(int32_t cols, int32_t rows, const int64_t *__restrict__ cptr,
-                                                      const int32_t *__restrict__ ridx,
-                                                      const double *__restrict__ val, double *__restrict__ dense) {
-  const int32_t j = blockIdx.x * 256 + threadIdx.x;
-  if (j >= cols) return;
-  for (int64_t e = cptr[j]; e < cptr[j + 1]; e++) dense[(int64_t)ridx[e] * cols + j] = val[e];
+// dense[r][j] = M3(r, j) from CCS (col_ptr over columns, row indices per entry), one wavefront
+// per column (Hubbard m = 396: 89 us with a thread per column, 7 with this).  serial: by its first lane alone, in stored order, for columns that hold a row
+// twice (the last value stays).
+__global__ __launch_bounds__(64) void k_ccs_to_dense(int32_t cols, const int64_t *__restrict__ cptr,
+                                                     const int32_t *__restrict__ ridx, const double *__restrict__ val,
+                                                     double *__restrict__ dense, int serial) {
+  const int32_t j = blockIdx.x;
+  const int step = serial ? 1 : 64;
+  if (serial && threadIdx.x > 0) return;
+  for (int64_t e = cptr[j] + threadIdx.x; e < cptr[j + 1]; e += step) dense[(int64_t)ridx[e] * cols + j] = val[e];
 }
 
 // out[i][j] = sum over the entries e of row i of A (stored order) of B[col_e][j] * A_e,
 // dropped to 0 when |sum| <= 1e-15; with skip_zero, terms whose B value is 0 are left out.
 // With kept set, the number of kept entries other than the last one, (rows-1, cols-1), is
-// added to *kept (the count the reference's capacity check sees, CRS_CRS_CCS_PRODUCT.c:56).
+// added to *kept (the count the reference's capacity check sees, CRS_CRS_CCS_PRODUCT.c:56);
+// with row_kept set, every row's number of kept entries to row_kept[row].
+// Waits for the loads of B, whose rows the entries pick: eight are in flight per thread, the
+// sum stays in stored order (Hubbard m = 396, T^dagger O T: 46 -> 40 and 63 -> 29 us a pass).
 template <bool kSkipZero>
 __global__ __launch_bounds__(256) void k_crs_dense(int32_t rows, int32_t cols, const int64_t *__restrict__ rptr,
                                                    const int32_t *__restrict__ cidx, const double *__restrict__ aval,
                                                    const double *__restrict__ B, double *__restrict__ out,
-                                                   unsigned long long *kept) {
+                                                   unsigned long long *kept, int32_t *row_kept) {
   const int32_t j = blockIdx.x * 256 + threadIdx.x;
+  const bool in = j < cols;
+  const int32_t jj = in ? j : cols - 1;
   unsigned int mine = 0;
-  if (j < cols) {
-    for (int32_t i = blockIdx.y; i < rows; i += gridDim.y) {
-      double s = 0.0;
-      for (int64_t e = rptr[i]; e < rptr[i + 1]; e++) {
-        const double b = B[(int64_t)cidx[e] * cols + j];
-        if (kSkipZero) {
-          if (b != 0.0) s = s + b * aval[e];
-        } else {
-          s = s + b * aval[e];
-        }
+  for (int32_t i = blockIdx.y; i < rows; i += gridDim.y) {
+    double s = 0.0;
+    const int64_t e1 = rptr[i + 1];
+    for (int64_t e = rptr[i]; e < e1; e += 8) {
+      double b[8], a[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        const int64_t q = e + u < e1 ? e + u : e1 - 1;
+        b[u] = B[(int64_t)cidx[q] * cols + jj];
+        a[u] = aval[q];
       }
-      const bool keep = std::fabs(s) > kDropBelow;
-      out[(int64_t)i * cols + j] = keep ? s : 0.0;
-      if (keep && !(i == rows - 1 && j == cols - 1)) mine++;
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        if (e + u < e1 && (!kSkipZero || b[u] != 0.0)) s = s + b[u] * a[u];
+    }
+    const bool keep = in && std::fabs(s) > kDropBelow;
+    if (in) out[(int64_t)i * cols + j] = keep ? s : 0.0;
+    if (keep && !(i == rows - 1 && j == cols - 1)) mine++;
+    if (row_kept) {
+      const int n = __popcll(__ballot(keep));
+      if ((threadIdx.x & 63) == 0 && n) atomicAdd(row_kept + i, n);
     }
   }
   if (!kept) return;   // uniform over the launch
@@ -72,6 +87,48 @@ __global__ __launch_bounds__(256) void k_crs_dense(int32_t rows, int32_t cols, c
   if (mine) atomicAdd(&cnt, mine);
   __syncthreads();
   if (threadIdx.x == 0 && cnt) atomicAdd(kept, (unsigned long long)cnt);
+}
+
+// Row pointers of the kept entries from their counts (one workgroup), and whether the last
+// entry, (rows-1, cols-1), is kept: rptr[rows + 1].
+__global__ __launch_bounds__(256) void k_row_pointers(int32_t rows, const int32_t *__restrict__ count,
+                                                      const double *__restrict__ out, int64_t last, int64_t *rptr) {
+  __shared__ int64_t sum[256];
+  const int32_t per = (rows + 255) / 256, b = min((int32_t)threadIdx.x * per, rows), e = min(b + per, rows);
+  int64_t mine = 0;
+  for (int32_t i = b; i < e; i++) mine += count[i];
+  sum[threadIdx.x] = mine;
+  __syncthreads();
+  int64_t at = 0;
+  for (int t = 0; t < (int)threadIdx.x; t++) at += sum[t];
+  for (int32_t i = b; i < e; i++) {
+    rptr[i] = at;
+    at += count[i];
+  }
+  if (threadIdx.x == 255) {
+    rptr[rows] = at;
+    rptr[rows + 1] = out[last] != 0.0;
+  }
+}
+
+// The kept entries of the dense result, columns ascending: one wavefront per row.
+__global__ __launch_bounds__(64) void k_compact_rows(int32_t rows, int32_t cols, const double *__restrict__ dense,
+                                                     const int64_t *__restrict__ rptr, int32_t *__restrict__ col,
+                                                     double *__restrict__ val) {
+  for (int32_t i = blockIdx.x; i < rows; i += gridDim.x) {
+    int64_t at = rptr[i];
+    for (int32_t j0 = 0; j0 < cols; j0 += 64) {
+      const int32_t j = j0 + threadIdx.x;
+      const double v = j < cols ? dense[(int64_t)i * cols + j] : 0.0;
+      const unsigned long long m = __ballot(v != 0.0);
+      if (v != 0.0) {
+        const int64_t q = at + __popcll(m & ((1ull << threadIdx.x) - 1));
+        col[q] = j;
+        val[q] = v;
+      }
+      at += __popcll(m);
+    }
+  }
 }
 
 void check_crs(const CRS1 *M, const char *what) {
@@ -107,68 +164,95 @@ void CRS_CRS_CCS_PRODUCT(CRS1 *M1, CRS1 *M2, CCS1 *M3, CRS1 *Out, CCS1 *Work, do
     const int64_t nnz3 = M3->Col[k];
     for (int32_t c = 0; c < k; c++)
       if (M3->Col[c] < 0 || M3->Col[c] > M3->Col[c + 1]) throw Failure(DMRGX_ERR_ARG, "M3 is not a valid CCS1");
-    for (int64_t e = 0; e < nnz3; e++)
-      if (M3->Row[e] < 0 || M3->Row[e] >= n3) throw Failure(DMRGX_ERR_ARG, "M3 is not a valid CCS1");
+    bool twice = false;   // a column of M3 that may hold a row twice
+    for (int32_t c = 0; c < k; c++)
+      for (int64_t e = M3->Col[c]; e < M3->Col[c + 1]; e++) {
+        if (M3->Row[e] < 0 || M3->Row[e] >= n3) throw Failure(DMRGX_ERR_ARG, "M3 is not a valid CCS1");
+        twice |= e > M3->Col[c] && M3->Row[e] <= M3->Row[e - 1];
+      }
     Context &C = ctx();
     hipStream_t st = C.stream;
     // M1's rows in ascending column order (the order pass 2 adds them in); a column stored
     // twice in a row keeps its last value, as the reference's dense scatter of the row does
     const int64_t nnz2 = M2->Row[n2];
-    std::vector<int64_t> hr1(n1 + 1, 0), perm;
+    bool sorted = true;
+    for (int32_t r = 0; r < n1 && sorted; r++)
+      for (int64_t e = M1->Row[r] + 1; e < M1->Row[r + 1]; e++)
+        if (M1->Col[e] <= M1->Col[e - 1]) {
+          sorted = false;
+          break;
+        }
+    std::vector<int64_t> hr1, perm;
     std::vector<int32_t> c1;
     std::vector<double> v1;
-    for (int32_t r = 0; r < n1; r++) {
-      const int64_t b = M1->Row[r], e = M1->Row[r + 1];
-      perm.resize(e - b);
-      std::iota(perm.begin(), perm.end(), b);
-      std::stable_sort(perm.begin(), perm.end(), [&](int64_t x, int64_t y) { return M1->Col[x] < M1->Col[y]; });
-      for (int64_t t = 0; t < e - b; t++) {
-        if (t + 1 < e - b && M1->Col[perm[t + 1]] == M1->Col[perm[t]]) continue;
-        c1.push_back(M1->Col[perm[t]]);
-        v1.push_back(M1->Val[perm[t]]);
+    const int64_t *p1 = reinterpret_cast<const int64_t *>(M1->Row);
+    const int32_t *q1 = M1->Col;
+    const double *a1 = M1->Val;
+    if (!sorted) {
+      hr1.assign(n1 + 1, 0);
+      for (int32_t r = 0; r < n1; r++) {
+        const int64_t b = M1->Row[r], e = M1->Row[r + 1];
+        perm.resize(e - b);
+        std::iota(perm.begin(), perm.end(), b);
+        std::stable_sort(perm.begin(), perm.end(), [&](int64_t x, int64_t y) { return M1->Col[x] < M1->Col[y]; });
+        for (int64_t t = 0; t < e - b; t++) {
+          if (t + 1 < e - b && M1->Col[perm[t + 1]] == M1->Col[perm[t]]) continue;
+          c1.push_back(M1->Col[perm[t]]);
+          v1.push_back(M1->Val[perm[t]]);
+        }
+        hr1[r + 1] = (int64_t)c1.size();
       }
-      hr1[r + 1] = (int64_t)c1.size();
+      p1 = hr1.data();
+      q1 = c1.data();
+      a1 = v1.data();
     }
-    const int64_t nnz1 = (int64_t)c1.size();
-    DevBuf<int64_t> r1(n1 + 1), r2(n2 + 1), p3(k + 1);
-    DevBuf<int32_t> dc1(nnz1 > 0 ? nnz1 : 1), dc2(nnz2 > 0 ? nnz2 : 1), dr3(nnz3 > 0 ? nnz3 : 1);
-    DevBuf<double> dv1(nnz1 > 0 ? nnz1 : 1), dv2(nnz2 > 0 ? nnz2 : 1), dv3(nnz3 > 0 ? nnz3 : 1);
     const int64_t nd3 = (int64_t)n3 * k, nw = (int64_t)n2 * k, no = (int64_t)n1 * k;
-    DevBuf<double> d3(nd3 > 0 ? nd3 : 1), w(nw > 0 ? nw : 1), o(no > 0 ? no : 1);
-    C.copy_in(r1.p, hr1.data(), sizeof(int64_t) * (n1 + 1));
-    C.copy_in(r2.p, M2->Row, sizeof(int64_t) * (n2 + 1));
-    C.copy_in(p3.p, M3->Col, sizeof(int64_t) * (k + 1));
-    if (nnz1 > 0) {
-      C.copy_in(dc1.p, c1.data(), sizeof(int32_t) * nnz1);
-      C.copy_in(dv1.p, v1.data(), sizeof(double) * nnz1);
-    }
-    if (nnz2 > 0) {
-      C.copy_in(dc2.p, M2->Col, sizeof(int32_t) * nnz2);
-      C.copy_in(dv2.p, M2->Val, sizeof(double) * nnz2);
-    }
-    if (nnz3 > 0) {
-      C.copy_in(dr3.p, M3->Row, sizeof(int32_t) * nnz3);
-      C.copy_in(dv3.p, M3->Val, sizeof(double) * nnz3);
-    }
-    std::vector<double> ho(no > 0 ? no : 1);
+    std::vector<int64_t> meta((size_t)n1 + 2, 0);   // row pointers of the result, last entry kept
     unsigned long long w_kept = 0;
+    DevBuf<int32_t> ocol;
+    DevBuf<double> oval;
+    DevBuf<char> mem;
     if (k > 0 && n1 > 0) {
-      DevBuf<unsigned long long> dkept(1);
-      HIPCHK(hipMemsetAsync(dkept.p, 0, sizeof(unsigned long long), st));
+      DevView<int64_t> r1, r2, p3;
+      DevView<int32_t> dc1, dc2, dr3, count;
+      DevView<double> dv1, dv2, dv3;
+      DevView<unsigned long long> dkept;
+      const std::vector<int32_t> zeros(n1, 0);
+      Upload up;
+      up.add(r1, p1, (size_t)n1 + 1);
+      up.add(dc1, q1, (size_t)p1[n1]);
+      up.add(dv1, a1, (size_t)p1[n1]);
+      up.add(r2, reinterpret_cast<const int64_t *>(M2->Row), (size_t)n2 + 1);
+      up.add(dc2, M2->Col, (size_t)nnz2);
+      up.add(dv2, M2->Val, (size_t)nnz2);
+      up.add(p3, reinterpret_cast<const int64_t *>(M3->Col), (size_t)k + 1);
+      up.add(dr3, M3->Row, (size_t)nnz3);
+      up.add(dv3, M3->Val, (size_t)nnz3);
+      up.add(count, zeros);
+      up.add(dkept, &w_kept, 1);
+      up.place(mem);
+      up.send();
+      DevBuf<double> d3(nd3 > 0 ? nd3 : 1), w(nw > 0 ? nw : 1), o(no);
+      DevBuf<int64_t> dmeta((size_t)n1 + 2);
       if (nd3 > 0) HIPCHK(hipMemsetAsync(d3.p, 0, sizeof(double) * nd3, st));
       const unsigned gx = (unsigned)((k + 255) / 256);
-      k_ccs_to_dense<<<gx, 256, 0, st>>>(k, n3, p3.p, dr3.p, dv3.p, d3.p);
+      k_ccs_to_dense<<<k, 64, 0, st>>>(k, p3.p, dr3.p, dv3.p, d3.p, twice ? 1 : 0);
       // grid y at most 65535; the kernels loop over the rows beyond it
       if (n2 > 0)
         k_crs_dense<false><<<dim3(gx, (unsigned)std::min(n2, 65535)), 256, 0, st>>>(n2, k, r2.p, dc2.p, dv2.p, d3.p,
-                                                                                   w.p, dkept.p);
+                                                                                   w.p, dkept.p, nullptr);
       k_crs_dense<true><<<dim3(gx, (unsigned)std::min(n1, 65535)), 256, 0, st>>>(n1, k, r1.p, dc1.p, dv1.p, w.p, o.p,
-                                                                                nullptr);
+                                                                                nullptr, count.p);
+      k_row_pointers<<<1, 256, 0, st>>>(n1, count.p, o.p, no - 1, dmeta.p);
       HIPCHK(hipGetLastError());
-      C.copy_out(ho.data(), o.p, sizeof(double) * no);
+      C.copy_out(meta.data(), dmeta.p, sizeof(int64_t) * meta.size());
       C.copy_out(&w_kept, dkept.p, sizeof(unsigned long long));
-    } else {
-      std::fill(ho.begin(), ho.end(), 0.0);
+      if (meta[n1] > 0) {
+        ocol.resize(meta[n1]);
+        oval.resize(meta[n1]);
+        k_compact_rows<<<(unsigned)std::min(n1, 65535), 64, 0, st>>>(n1, k, o.p, dmeta.p, ocol.p, oval.p);
+        HIPCHK(hipGetLastError());
+      }
     }
     // The reference checks the kept count against the capacity before every entry it
     // evaluates (CRS_CRS_CCS_PRODUCT.c:56 for Work, :101 for Out), so it exits when the
@@ -176,25 +260,14 @@ void CRS_CRS_CCS_PRODUCT(CRS1 *M1, CRS1 *M2, CCS1 *M3, CRS1 *Out, CCS1 *Work, do
     // is stored after them.
     if (n2 > 0 && k > 0 && (long long)w_kept >= (long long)Work->max_val)
       throw Failure(DMRGX_ERR_ARG, "Work has too few elements");
-    if (n1 > 0 && k > 0) {
-      long long out_kept = 0;
-      for (int64_t t = 0; t + 1 < no; t++) out_kept += ho[t] != 0.0;
-      if (out_kept >= (long long)Out->max_val) throw Failure(DMRGX_ERR_ARG, "Out has too few elements");
-    }
-    // compaction into Out, columns ascending (sml/CRS_CRS_CCS_PRODUCT.c:98-121)
-    int64_t e = 0;
-    Out->Row[0] = 0;
-    for (int32_t i = 0; i < n1; i++) {
-      for (int32_t j = 0; j < k; j++) {
-        const double v = ho[(int64_t)i * k + j];
-        if (v != 0.0) {
-          if (e >= Out->max_val) throw Failure(DMRGX_ERR_ARG, "Out has too few elements");
-          Out->Val[e] = v;
-          Out->Col[e] = j;
-          e++;
-        }
-      }
-      Out->Row[i + 1] = e;
+    if (n1 > 0 && k > 0 && meta[n1] - meta[n1 + 1] >= (int64_t)Out->max_val)
+      throw Failure(DMRGX_ERR_ARG, "Out has too few elements");
+    if (meta[n1] > (int64_t)Out->max_val) throw Failure(DMRGX_ERR_ARG, "Out has too few elements");
+    // Out, columns ascending (sml/CRS_CRS_CCS_PRODUCT.c:98-121)
+    for (int32_t i = 0; i <= n1; i++) Out->Row[i] = (long)meta[i];
+    if (meta[n1] > 0) {
+      C.copy_out(Out->Val, oval.p, sizeof(double) * meta[n1]);
+      C.copy_out(Out->Col, ocol.p, sizeof(int32_t) * meta[n1]);
     }
     Out->row_dim = n1;
     Out->col_dim = k;
