@@ -325,6 +325,8 @@ static dmrgx_superblock *create_superblock(int32_t n, int32_t dim_LL, int32_t di
     const int64_t nnz = a.row[a.row_dim] - a.row[0];
     for (int64_t j = 0; j < nnz; j++)
       if (a.col[j] < 0 || a.col[j] >= op_col_limit[i]) throw Failure(DMRGX_ERR_ARG, "operator column outside its block");
+    for (int32_t r = 0; r < a.row_dim; r++)
+      for (int64_t j = a.row[r] + 1; j < a.row[r + 1]; j++) S->ascending &= a.col[j] > a.col[j - 1];
   }
   S->nt = (int)terms.size();
   S->hterms = terms;

@@ -117,6 +117,54 @@ __global__ __launch_bounds__(256) void k_kron_right(KronBuild kb, const DTerm *t
   }
 }
 
+// The same rows with one wavefront per state and the row in LDS, its lanes over the (op1 entry,
+// op2 entry) products of a term.  Within a term no two products reach one state (the operators'
+// rows hold a column once: dmrgx_superblock::ascending; otherwise, or for a row above
+// kHalfRow states, the kernels above), and a wavefront's LDS accesses are in order, so
+// every element sums the same products in the same order.  The kernels above wait for a chain of
+// some thousand dependent loads: KLM m = 799 479 + 468 us, Hubbard m = 396 231 + 258; this one
+// takes 41 + 38 and below 20 + 20.
+constexpr int kHalfRow = 2048;
+template <bool kLeft>
+__global__ __launch_bounds__(256) void k_kron_half(KronBuild kb, const DTerm *terms, const int32_t *ids, int nt,
+                                                   const DOp *ops, const int32_t *const *eles, double *M) {
+  __shared__ double rows[4][kHalfRow];
+  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int32_t i = blockIdx.x * 4 + wave;
+  if (i >= (kLeft ? kb.nstate_a : kb.nstate_b)) return;   // no barrier below
+  const int32_t *sec = kLeft ? kb.asec : kb.bsec, *idx = kLeft ? kb.aidx : kb.bidx;
+  const int s = sec[i];
+  const KronSector S = kb.sec[s];
+  const int32_t first = kLeft ? S.a0 : S.b0, dim = kLeft ? S.da : S.db;
+  const int block = kLeft ? kb.aLL[i] : kb.bRR[i], site = kLeft ? kb.aLR[i] : kb.bRL[i];
+  const int q[4] = {kLeft ? block : 0, kLeft ? site : 0, kLeft ? 0 : block, kLeft ? 0 : site};
+  double *row = rows[wave];
+  for (int32_t c = l; c < dim; c += 64) row[c] = 0.0;
+  __builtin_amdgcn_wave_barrier();
+  for (int u = 0; u < nt; u++) {
+    const DTerm t = terms[ids[u]];
+    const DOp a = ops[t.op1], b = t.s2 < 0 ? a : ops[t.op2];
+    const double sc = (double)term_sign(t, eles, q) * t.coeff;
+    const int64_t b1 = a.row[q[t.s1]], n1 = a.row[q[t.s1] + 1] - b1;
+    const int64_t b2 = t.s2 < 0 ? 0 : b.row[q[t.s2]], n2 = t.s2 < 0 ? 1 : b.row[q[t.s2] + 1] - b2;
+    for (int64_t e = l; e < n1 * n2; e += 64) {
+      const int64_t i1 = e / n2, i2 = e - i1 * n2;
+      int st[2] = {block, site};
+      st[t.s1 & 1] = a.col[b1 + i1];
+      double p = sc * a.val[b1 + i1];
+      if (t.s2 >= 0) {
+        st[t.s2 & 1] = b.col[b2 + i2];
+        p = p * b.val[b2 + i2];
+      }
+      const int32_t c = idx[st[0] * kb.d + st[1]];
+      if (c >= 0 && sec[c] == s && fabs(p) > 1.0e-15) row[c - first] += p;
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  double *out = M + (kLeft ? S.ml : S.mr);
+  for (int32_t c = l; c < dim; c += 64) out[kron_at(i - first, c, dim)] = row[c];
+}
+
 // zc = coupling terms applied to x, the general form (KronDev::general).  A coupling term has
 // one operator on each half (op1 on LL or LR, op2 on RR or RL) and a sign that is a product of a
 // factor of the row's LLLR state and one of its RRRL state, so per term the builder lists,
@@ -523,12 +571,20 @@ int dmrgx_superblock_kron(const dmrgx_superblock *S, dmrgx_kron **out) {
     k_zero<<<1024, 256, 0, st>>>(ml, K.ML.p);
     k_zero<<<1024, 256, 0, st>>>(mr, K.MR.p);
     const KronBuild kb{d, K.na, K.nb, daLL.p, daLR.p, dbRR.p, dbRL.p, K.asec.p, K.bsec.p, K.aidx.p, K.bidx.p, K.sec.p};
-    if (K.na > 0)
-      k_kron_left<<<(K.na + 255) / 256, 256, 0, st>>>(kb, S->terms.p, dleft.p, (int)left.size(), S->ops.p,
-                                                      S->ele_ptrs.p, K.ML.p);
-    if (K.nb > 0)
-      k_kron_right<<<(K.nb + 255) / 256, 256, 0, st>>>(kb, S->terms.p, dright.p, (int)right.size(), S->ops.p,
-                                                       S->ele_ptrs.p, K.MR.p);
+    int32_t widest = 0;
+    for (const KronSector &sc : K.hsec) widest = std::max({widest, sc.da, sc.db});
+    const int nl = (int)left.size(), nr = (int)right.size();
+#define HALF_ARGS(ids, n, M) kb, S->terms.p, ids.p, n, S->ops.p, S->ele_ptrs.p, M.p
+    if (K.na > 0 && K.nb > 0) {
+      if (S->ascending && widest <= kHalfRow) {
+        k_kron_half<true><<<(K.na + 3) / 4, 256, 0, st>>>(HALF_ARGS(dleft, nl, K.ML));
+        k_kron_half<false><<<(K.nb + 3) / 4, 256, 0, st>>>(HALF_ARGS(dright, nr, K.MR));
+      } else {
+        k_kron_left<<<(K.na + 255) / 256, 256, 0, st>>>(HALF_ARGS(dleft, nl, K.ML));
+        k_kron_right<<<(K.nb + 255) / 256, 256, 0, st>>>(HALF_ARGS(dright, nr, K.MR));
+      }
+    }
+#undef HALF_ARGS
     HIPCHK(hipGetLastError());
     *out = H.release();   // no wait: the host lists have been read, products queue behind the build
   });

@@ -68,6 +68,7 @@ struct dmrgx_superblock {
   dmrgx::DevView<dmrgx::DOp> ops;
   dmrgx::DevView<dmrgx::DTerm> terms;
   dmrgx::DevView<const int32_t *> ele_ptrs;
+  bool ascending = true;   // every operator's rows hold ascending columns, none twice
   // host copies of the operators of the coupling terms (for the Kronecker form's state lists)
   struct HostOp {
     std::vector<int64_t> row;

@@ -212,3 +212,33 @@ def test_gpu_kron_tile_edges(left, right, far, variant):
         K.free()
         sb.free()
 
+
+
+@pytest.mark.gpu
+def test_gpu_kron_repeated_operator_columns():
+    """Operators whose rows hold columns out of order and twice (both entries count, as the element
+    makers add them): the sector matrices' general build."""
+    import dmrg_c_amd as D
+    import oracle_py as O
+    import scipy.sparse as sp
+    from dmrg_c_amd import snapshot as S
+    s = _random_superblock([3, 12, 5], [2, 14, 3], True, 9)
+    for k in (0, 5, 6):
+        o = s.ops[k]
+        rows = [list(zip(o.col[a:b], o.val[a:b])) for a, b in zip(o.row[:-1], o.row[1:])]
+        rows = [[(c, 0.25 * v) for c, v in r] + [(c, 0.75 * v) for c, v in reversed(r)] for r in rows]
+        flat = [e for r in rows for e in r]
+        s.ops[k] = S.Crs(o.row_dim, o.col_dim, np.cumsum([0] + [len(r) for r in rows]).astype(np.int64),
+                         np.array([c for c, _ in flat], np.int32), np.array([v for _, v in flat]))
+    row, col, val = O.assemble(s)
+    A = sp.csr_matrix((val, col, row), shape=(s.n, s.n))
+    A = (A + A.T - sp.diags(A.diagonal())).tocsr()
+    sb = D.Superblock(s)
+    K = sb.kron()
+    try:
+        x = np.random.default_rng(3).standard_normal(s.n)
+        y = K.matvec(x)
+        assert np.abs(y - A @ x).max() <= 1e-13 * np.abs(x).max() * abs(A).sum(axis=1).max()
+    finally:
+        K.free()
+        sb.free()
