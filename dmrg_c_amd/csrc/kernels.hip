@@ -1171,20 +1171,28 @@ void Reduce::ensure(size_t blocks) {
   if (partial.count < blocks) partial.resize(blocks);
 }
 
+// Lanes per row of a CSR matrix.  A gather instruction touches fewer lines the more rows it
+// covers at like places, so few lanes win as long as the chip is full: 4 for rows of a dozen
+// entries, 16 above (8 would be a few percent faster still in large matrices, but every lane
+// then sums twice as long a chain, with that much more rounding).  Product and dot, microseconds,
+// at the old rule (a third of the row length, up to 64) and with 4 / 8 / 16 lanes: XXZ m = 162
+// (n = 23524, 164 a row) 21.9 and 13.9 / 12.6 / 13.2; Hubbard m = 250 (56244, 115) 43 and 20.3 /
+// 19.3 / 19.0; Hubbard m = 396 (144542, 186) 151 and 76 / 71 / 76; KLM m = 300 (287520, 131) 254 and
+// 114 / 107 / 120; KLM m = 60 (12870, 30) 7.4 and 6.1 / 6.3 / 6.4; XXZ m = 30 (790, 29) 5.6 and
+// 5.9 / 5.7 / 5.4; ED XXZ L = 20 (184756, 11) 14.0 and 10.5 / 14.2 / 21.8.
 int pick_lanes(int32_t n, int64_t nnz) {
   const double avg = n > 0 ? (double)nnz / n : 0.0;
-  int g = 4;
-  while (g < 64 && g * 3 < avg) g <<= 1;
-  return g;
+  return avg < 12.0 ? 4 : 16;
 }
 
 void default_schedule(dmrgx_matrix &A) {
   A.lanes = pick_lanes(A.n, A.nnz);
   A.grid = kGridCap;
-  // eight loads in flight per lane; the value dictionary only where the tuner finds it
-  // faster (its table lookups cost more than the 4 bytes per entry they save on MI355X for
-  // the superblocks measured)
-  A.load = kLoadDeep;
+  // eight loads in flight per lane where a lane has that many entries (in shorter rows the
+  // positions past the end load the last entry again: ED XXZ L = 18, 10 a row, 7.1 against 6.3 us);
+  // the value dictionary only where the tuner finds it faster (its table lookups cost more
+  // than the 4 bytes per entry they save on MI355X for the superblocks measured)
+  A.load = (double)A.nnz >= 12.0 * A.lanes * A.n ? kLoadDeep : 0;
 }
 
 int spmv_blocks(int32_t n, int lanes, int grid_cap) {
