@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <numeric>
 #include <vector>
 
@@ -207,16 +208,16 @@ void CRS_CRS_CCS_PRODUCT(CRS1 *M1, CRS1 *M2, CCS1 *M3, CRS1 *Out, CCS1 *Work, do
       a1 = v1.data();
     }
     const int64_t nd3 = (int64_t)n3 * k, nw = (int64_t)n2 * k, no = (int64_t)n1 * k;
-    std::vector<int64_t> meta((size_t)n1 + 2, 0);   // row pointers of the result, last entry kept
-    unsigned long long w_kept = 0;
-    DevBuf<int32_t> ocol;
-    DevBuf<double> oval;
-    DevBuf<char> mem;
+    // the result's row pointers, whether its last entry is kept, the entries kept of W; then, on the
+    // device behind them, its values and columns
+    std::vector<int64_t> meta((size_t)n1 + 3, 0);
+    const size_t meta_bytes = sizeof(int64_t) * meta.size();
+    std::vector<char> all;   // a small result, copied back whole with its pointers
+    DevBuf<char> mem, result;
     if (k > 0 && n1 > 0) {
       DevView<int64_t> r1, r2, p3;
       DevView<int32_t> dc1, dc2, dr3, count;
       DevView<double> dv1, dv2, dv3;
-      DevView<unsigned long long> dkept;
       const std::vector<int32_t> zeros(n1, 0);
       Upload up;
       up.add(r1, p1, (size_t)n1 + 1);
@@ -229,45 +230,55 @@ void CRS_CRS_CCS_PRODUCT(CRS1 *M1, CRS1 *M2, CCS1 *M3, CRS1 *Out, CCS1 *Work, do
       up.add(dr3, M3->Row, (size_t)nnz3);
       up.add(dv3, M3->Val, (size_t)nnz3);
       up.add(count, zeros);
-      up.add(dkept, &w_kept, 1);
       up.place(mem);
       up.send();
       DevBuf<double> d3(nd3 > 0 ? nd3 : 1), w(nw > 0 ? nw : 1), o(no);
-      DevBuf<int64_t> dmeta((size_t)n1 + 2);
+      result.resize(meta_bytes + (sizeof(double) + sizeof(int32_t)) * (size_t)no);
+      int64_t *dmeta = reinterpret_cast<int64_t *>(result.p);
+      double *oval = reinterpret_cast<double *>(result.p + meta_bytes);
+      int32_t *ocol = reinterpret_cast<int32_t *>(oval + no);
+      unsigned long long *dkept = reinterpret_cast<unsigned long long *>(dmeta + n1 + 2);
+      HIPCHK(hipMemsetAsync(dkept, 0, sizeof(unsigned long long), st));
       if (nd3 > 0) HIPCHK(hipMemsetAsync(d3.p, 0, sizeof(double) * nd3, st));
       const unsigned gx = (unsigned)((k + 255) / 256);
       k_ccs_to_dense<<<k, 64, 0, st>>>(k, p3.p, dr3.p, dv3.p, d3.p, twice ? 1 : 0);
       // grid y at most 65535; the kernels loop over the rows beyond it
       if (n2 > 0)
         k_crs_dense<false><<<dim3(gx, (unsigned)std::min(n2, 65535)), 256, 0, st>>>(n2, k, r2.p, dc2.p, dv2.p, d3.p,
-                                                                                   w.p, dkept.p, nullptr);
+                                                                                   w.p, dkept, nullptr);
       k_crs_dense<true><<<dim3(gx, (unsigned)std::min(n1, 65535)), 256, 0, st>>>(n1, k, r1.p, dc1.p, dv1.p, w.p, o.p,
                                                                                 nullptr, count.p);
-      k_row_pointers<<<1, 256, 0, st>>>(n1, count.p, o.p, no - 1, dmeta.p);
+      k_row_pointers<<<1, 256, 0, st>>>(n1, count.p, o.p, no - 1, dmeta);
+      k_compact_rows<<<(unsigned)std::min(n1, 65535), 64, 0, st>>>(n1, k, o.p, dmeta, ocol, oval);
       HIPCHK(hipGetLastError());
-      C.copy_out(meta.data(), dmeta.p, sizeof(int64_t) * meta.size());
-      C.copy_out(&w_kept, dkept.p, sizeof(unsigned long long));
-      if (meta[n1] > 0) {
-        ocol.resize(meta[n1]);
-        oval.resize(meta[n1]);
-        k_compact_rows<<<(unsigned)std::min(n1, 65535), 64, 0, st>>>(n1, k, o.p, dmeta.p, ocol.p, oval.p);
-        HIPCHK(hipGetLastError());
+      // small results: all of the buffer in one copy, rather than a wait for the count before a second
+      if (result.count <= 256 * 1024) {
+        all.resize(result.count);
+        C.copy_out(all.data(), result.p, all.size());
+        std::memcpy(meta.data(), all.data(), meta_bytes);
+      } else {
+        C.copy_out(meta.data(), result.p, meta_bytes);
       }
     }
+    const long long w_kept = meta[n1 + 2];
     // The reference checks the kept count against the capacity before every entry it
     // evaluates (CRS_CRS_CCS_PRODUCT.c:56 for Work, :101 for Out), so it exits when the
     // entries kept before the last evaluated position reach max_val, even if nothing more
     // is stored after them.
-    if (n2 > 0 && k > 0 && (long long)w_kept >= (long long)Work->max_val)
+    if (n2 > 0 && k > 0 && w_kept >= (long long)Work->max_val)
       throw Failure(DMRGX_ERR_ARG, "Work has too few elements");
     if (n1 > 0 && k > 0 && meta[n1] - meta[n1 + 1] >= (int64_t)Out->max_val)
       throw Failure(DMRGX_ERR_ARG, "Out has too few elements");
     if (meta[n1] > (int64_t)Out->max_val) throw Failure(DMRGX_ERR_ARG, "Out has too few elements");
     // Out, columns ascending (sml/CRS_CRS_CCS_PRODUCT.c:98-121)
     for (int32_t i = 0; i <= n1; i++) Out->Row[i] = (long)meta[i];
-    if (meta[n1] > 0) {
-      C.copy_out(Out->Val, oval.p, sizeof(double) * meta[n1]);
-      C.copy_out(Out->Col, ocol.p, sizeof(int32_t) * meta[n1]);
+    const size_t nz = (size_t)meta[n1], col_at = meta_bytes + sizeof(double) * (size_t)no;
+    if (nz > 0 && !all.empty()) {
+      std::memcpy(Out->Val, all.data() + meta_bytes, sizeof(double) * nz);
+      std::memcpy(Out->Col, all.data() + col_at, sizeof(int32_t) * nz);
+    } else if (nz > 0) {
+      C.copy_out(Out->Val, result.p + meta_bytes, sizeof(double) * nz);
+      C.copy_out(Out->Col, result.p + col_at, sizeof(int32_t) * nz);
     }
     Out->row_dim = n1;
     Out->col_dim = k;
