@@ -1064,17 +1064,43 @@ __global__ __launch_bounds__(64) void k_tri_fill(int32_t n, const int64_t *__res
   }
 }
 
-// One wavefront per row: sort the row's tail records by column (the columns are
-// distinct) and write them after the row's own entries.  Tails up to kTailCap entries are
-// bitonic-sorted in LDS; longer ones by one lane.
+// One wavefront per row: put the row's tail records in column order (the columns are
+// distinct) after the row's own entries.  Tails up to kTailCap entries go straight to their
+// rank, the number of smaller columns of the tail, counted against all of them in LDS (four a
+// load, the same for every lane).  A bitonic network in LDS needs a barrier after each of its
+// log^2 steps and moves the values along (Hubbard m = 396: 439 us; this 161).  Longer tails are
+// inserted one by one.
 constexpr int kTailCap = 512;
+template <int U>
+__device__ __forceinline__ void rank_tail(const int4 *kc, int m, const TailRec *__restrict__ src, int64_t b,
+                                          int32_t *__restrict__ fcol, double *__restrict__ fval) {
+  int32_t c[U], rank[U];
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const int i = threadIdx.x + 64 * u;
+    c[u] = i < m ? src[i].col : -1;
+    rank[u] = 0;
+  }
+  for (int j = 0; j < (m + 3) / 4; j++) {
+    const int4 o = kc[j];
+#pragma unroll
+    for (int u = 0; u < U; u++) rank[u] += (int)(o.x < c[u]) + (int)(o.y < c[u]) + (int)(o.z < c[u]) + (int)(o.w < c[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const int i = threadIdx.x + 64 * u;
+    if (i < m) {
+      fcol[b + rank[u]] = c[u];
+      fval[b + rank[u]] = src[i].val;
+    }
+  }
+}
 __global__ __launch_bounds__(64) void k_sort_tail(int32_t n, const int64_t *__restrict__ trow,
                                                   const int64_t *__restrict__ frow,
                                                   const TailRec *__restrict__ tail,
                                                   int32_t *__restrict__ fcol,
                                                   double *__restrict__ fval) {
-  __shared__ int32_t kc[kTailCap];
-  __shared__ double kv[kTailCap];
+  __shared__ int4 kc[kTailCap / 4];
   const int32_t r = blockIdx.x;
   if (r >= n) return;
   const int lane = threadIdx.x;
@@ -1099,42 +1125,12 @@ __global__ __launch_bounds__(64) void k_sort_tail(int32_t n, const int64_t *__re
     }
     return;
   }
-  int P = 1;
-  while (P < m) P <<= 1;
-  for (int i = lane; i < P; i += 64) {
-    if (i < m) {
-      const TailRec t = src[i];
-      kc[i] = t.col;
-      kv[i] = t.val;
-    } else {
-      kc[i] = INT32_MAX;
-      kv[i] = 0.0;
-    }
-  }
+  for (int i = lane; i < (m + 3) / 4 * 4; i += 64) reinterpret_cast<int32_t *>(kc)[i] = i < m ? src[i].col : INT32_MAX;
   __syncthreads();
-  for (int size = 2; size <= P; size <<= 1) {
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int i = lane; i < P; i += 64) {
-        const int jx = i ^ stride;
-        if (jx > i) {
-          const bool up = (i & size) == 0;
-          const int32_t x = kc[i], y = kc[jx];
-          if ((x > y) == up) {
-            kc[i] = y;
-            kc[jx] = x;
-            const double t = kv[i];
-            kv[i] = kv[jx];
-            kv[jx] = t;
-          }
-        }
-      }
-      __syncthreads();
-    }
-  }
-  for (int i = lane; i < m; i += 64) {
-    fcol[b + i] = kc[i];
-    fval[b + i] = kv[i];
-  }
+  if (m <= 64) rank_tail<1>(kc, m, src, b, fcol, fval);
+  else if (m <= 128) rank_tail<2>(kc, m, src, b, fcol, fval);
+  else if (m <= 256) rank_tail<4>(kc, m, src, b, fcol, fval);
+  else rank_tail<8>(kc, m, src, b, fcol, fval);
 }
 
 __global__ __launch_bounds__(kBlock) void k_to_fp32(int64_t nnz, const double *__restrict__ v,
@@ -1297,9 +1293,9 @@ int residual_l1_default_blocks(int32_t n, int64_t nnz) { return spmv_blocks(n, p
 
 void launch_residual_l1_into(int32_t n, int64_t nnz, const int64_t *row, const int32_t *col, const double *val,
                              const double *v, double eig, double *out, double *partial, hipStream_t s) {
-  // default_schedule's choices for a CSR matrix of these dimensions (lanes from the mean row
-  // length, kGridCap workgroups, eight loads in flight, CSR), so that the result equals
-  // launch_residual_l1 on a dmrgx_matrix of the same arrays bit for bit
+  // default_schedule's lanes and workgroups for a CSR matrix of these dimensions, so that the
+  // result equals launch_residual_l1 on a dmrgx_matrix of the same arrays bit for bit (the loads
+  // in flight do not change the order of the sums)
   apply_rows_into(n, pick_lanes(n, nnz), kGridCap, CsrRows<double, kLoadDeep>{row, col, val, nnz}, v,
                   EpiResidualL1{v, out, eig}, partial, s, 0, true, false);
 }

@@ -242,3 +242,37 @@ def test_big_superblock_assembly_and_solve(name):
     e_ref = float(s.meta["gs_energy"][0])
     assert abs(E - e_ref) <= 1e-10 * abs(e_ref), (E, e_ref)
     assert st.gs_error < 1e-9
+
+
+def test_expand_tail_lengths():
+    """The symmetric expansion's rows for every tail length at which its sort changes over: 0, the
+    ends of 64, 128 and 256 entries, and past 512, where the tail is inserted one by one."""
+    lengths = [0, 1, 2, 3, 4, 5, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 600]
+    n, rng = 700, np.random.default_rng(5)
+    L = np.zeros((n, n), bool)
+    for c, m in enumerate(lengths):
+        L[rng.choice(np.arange(c + 1, n), m, replace=False), c] = True
+    np.fill_diagonal(L, True)
+    row = np.concatenate([[0], np.cumsum(L.sum(1))]).astype(np.int64)
+    col = np.nonzero(L)[1].astype(np.int32)
+    val = rng.standard_normal(len(col))
+    A = D.DeviceMatrix(row, col, val)
+    got, ref = A.download(), O.expand_sym(n, row, col, val)
+    A.free()
+    for g, r in zip(got, ref):
+        assert np.array_equal(g, r)
+
+
+@pytest.mark.parametrize("left,right", [([1], [1]), ([30, 33], [31, 35]), ([60, 70], [66, 64]), ([120, 140], [4, 3])])
+def test_assembly_list_lengths(left, right):
+    """Rows of 1 to 266 entries: contribution lists on both sides of every length at which the
+    assembly's sort changes over, and past the short list's capacity; identical to the oracle."""
+    from test_kron import _random_superblock
+    s = _random_superblock(left, right, True, 11)
+    sb = D.Superblock(s)
+    sb.assemble(full=False)
+    row, col, val = sb.download_lower()
+    orow, ocol, oval = O.assemble(s)
+    sb.free()
+    assert np.array_equal(row, orow) and np.array_equal(col, ocol)
+    assert np.array_equal(val.view(np.int64), oval.view(np.int64))
