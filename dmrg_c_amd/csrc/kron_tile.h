@@ -56,11 +56,11 @@ struct KronFrag {
 // the slab, plus an offset of the lane that the loop does not change (hence the shifted last slab,
 // kron_slab: no clamping at the edge).
 //
-// Measured (MI355X, KLM m = 799: 3.23 GFLOP a product, 2133 tiles of 32 x 32): 81 us, of which the
-// matrix cores are busy 46; the two products by a kernel of 64 x 64 LDS-staged tiles, the coupling
-// terms on a side stream and the epilogue by a third kernel took 110 us together.  Wider tiles
-// of a wavefront (32 x 64, 64 x 64) read less but gave 85 and 105 us: fewer of them fit.  Hubbard
-// m = 396 (68 MFLOP, 641 tiles of 16 x 16): 9 us against 31, all of it latency.
+// Measured (MI355X, KLM m = 799: 3.23 GFLOP a product, 2133 tiles of 32 x 32): 88 us with the Lanczos
+// epilogue and 72 with CG's, of which the matrix cores are busy 46; 64 x 64 LDS-staged tiles took 86 us
+// and the epilogue's own kernel 14 to 25 more, with the coupling terms on a side stream.  Whole
+// solves by tile: 32 x 32 83 ms, 32 x 64 84 to 87 ms, 64 x 64 101 to 107 ms.  Hubbard m = 396
+// (68 MFLOP, 641 tiles of 16 x 16): 9 us against 30, most of it latency.
 //
 // M_L and M_R are zero where a shifted last slab repeats a k or a sector is narrower than a slab
 // (X's operand there is its last row or column again), and in rows beyond the sector.
