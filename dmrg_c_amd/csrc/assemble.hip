@@ -45,6 +45,21 @@ __device__ __forceinline__ unsigned lanes_below(uint64_t mask) {
   return __popcll(mask & ((1ull << (threadIdx.x & 63)) - 1ull));
 }
 
+// a[s] without an indexed register array (s differs from lane to lane)
+template <class T>
+__device__ __forceinline__ T slot_of(const T (&a)[4], int s) {
+  return s == 0 ? a[0] : s == 1 ? a[1] : s == 2 ? a[2] : a[3];
+}
+template <class T>
+__device__ __forceinline__ const T *shfl_ptr(const T *p, int l) {
+  return reinterpret_cast<const T *>(__shfl((unsigned long long)reinterpret_cast<uintptr_t>(p), l));
+}
+// lane l's v as a wave-uniform value
+__device__ __forceinline__ int64_t read_lane(int64_t v, int l) {
+  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)v, l), hi = __builtin_amdgcn_readlane((uint32_t)((uint64_t)v >> 32), l);
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
 // Puts the m <= 64 U distinct keys of one wavefront in ascending order, each straight to its
 // rank: the number of smaller keys, counted against all of them in LDS (two a load, the same for
 // every lane).  key[m] is past the end and larger than all if m is odd.  A bitonic network
@@ -94,38 +109,79 @@ __global__ __launch_bounds__(64) void k_assemble(SbView sb, const int32_t *row_l
   const int32_t r = row_list ? row_list[item] : item;
   const int q[4] = {sb.LL[r], sb.LR[r], sb.RR[r], sb.RL[r]};
   int m = 0;  // list length (wave-uniform)
-  for (int t = 0; t < sb.nt; t++) {
-    const DTerm tm = sb.terms[t];
-    if (tm.kind == K_ZERO) continue;  // handled after the sums (see file comment)
-    const DOp a = sb.ops[tm.op1];
-    const int64_t b1 = a.row[q[tm.s1]];
-    const int64_t l1 = a.row[q[tm.s1] + 1] - b1;
-    int64_t b2 = 0, l2 = 1;
-    DOp b = a;
-    if (tm.s2 >= 0) {
-      b = sb.ops[tm.op2];
-      b2 = b.row[q[tm.s2]];
-      l2 = b.row[q[tm.s2] + 1] - b2;
+  const int64_t stride[4] = {(int64_t)sb.d * sb.dim_RR * sb.d, (int64_t)sb.dim_RR * sb.d, sb.d, 1};
+  const int64_t at_r = sb_index(q[0], q[1], q[2], q[3], sb.dim_RR, sb.d);
+  // Up to 64 terms at a time: lane t first holds term t (its operators' rows, sign and
+  // number of contributions), then the lanes go over all their contributions one after another,
+  // in list order, each fetching its term's data from the lane that holds it.  Term by term, each
+  // term's few contributions waited for its row bounds, columns and inverse in turn (count pass,
+  // Hubbard m = 396: 549 us; this 495, at 77 registers; held to 64 it spills and takes 544).
+  for (int t0 = 0; t0 < sb.nt; t0 += 64) {
+    const int32_t *col1 = nullptr, *col2 = nullptr;
+    const double *val1 = nullptr, *val2 = nullptr;
+    int64_t l2 = 1, total = 0, st1 = 0, st2 = 0, origin = at_r;
+    double sc = 0.0;
+    const int nt = min(64, sb.nt - t0);
+    if (lane < nt) {
+      const DTerm tm = sb.terms[t0 + lane];
+      if (tm.kind != K_ZERO) {  // ZERO: handled after the sums (see file comment)
+        const DOp o = sb.ops[tm.op1];
+        const int q1 = slot_of(q, tm.s1);
+        const int64_t b1 = o.row[q1];
+        total = o.row[q1 + 1] - b1;
+        col1 = o.col + b1;
+        val1 = o.val + b1;
+        st1 = slot_of(stride, tm.s1);
+        origin -= q1 * st1;
+        if (tm.s2 >= 0) {
+          const DOp o2 = sb.ops[tm.op2];
+          const int q2 = slot_of(q, tm.s2);
+          const int64_t b2 = o2.row[q2];
+          l2 = o2.row[q2 + 1] - b2;
+          total *= l2;
+          col2 = o2.col + b2;
+          val2 = o2.val + b2;
+          st2 = slot_of(stride, tm.s2);
+          if (tm.s2 == tm.s1) st1 = 0;   // the second operator's column counts
+          else origin -= q2 * st2;
+        }
+        if (total > 0) sc = (double)term_sign(tm, sb.eles, q) * tm.coeff;
+      }
     }
-    const int64_t total = l1 * l2;
-    if (total == 0) continue;
-    const double sc = (double)term_sign(tm, sb.eles, q) * tm.coeff;
-    for (int64_t base = 0; base < total; base += 64) {
-      const int64_t k = base + lane;
+    int64_t end = total;   // contributions of the terms up to this lane's
+    for (int s = 1; s < 64; s <<= 1) {
+      const int64_t below = __shfl_up(end, s);
+      if (lane >= s) end += below;
+    }
+    const int64_t first = end - total;
+    const int64_t all = read_lane(end, 63);
+    for (int64_t base = 0; base < all; base += 64) {
+      const int64_t f = base + lane;
+      // the last term that begins at or before f (of several the last: the others are empty)
+      int t = 0;
+      for (int s = 32; s > 0; s >>= 1) {
+        const int64_t b = __shfl(first, (t + s) & 63);
+        if (t + s < nt && b <= f) t += s;
+      }
+      const int64_t k = f - __shfl(first, t), len2 = __shfl(l2, t);
+      const int32_t *c1 = shfl_ptr(col1, t), *c2 = shfl_ptr(col2, t);
+      const double *v1 = shfl_ptr(val1, t), *v2 = shfl_ptr(val2, t);
+      const int64_t s1 = __shfl(st1, t), s2 = __shfl(st2, t), o = __shfl(origin, t);
+      const double sign = __shfl(sc, t);
       bool keep = false;
       int32_t col = 0;
       double v = 0.0;
-      if (k < total) {
-        int qq[4] = {q[0], q[1], q[2], q[3]};
-        const int64_t i = (tm.s2 >= 0) ? k / l2 : k;
-        qq[tm.s1] = a.col[b1 + i];
-        double prod = sc * a.val[b1 + i];
-        if (tm.s2 >= 0) {
-          const int64_t j = k - i * l2;
-          qq[tm.s2] = b.col[b2 + j];
-          prod = prod * b.val[b2 + j];
+      if (f < all) {
+        int64_t i = k;
+        if (len2 > 1) i = ((uint64_t)(k | len2) >> 32) ? k / len2 : (int64_t)((uint32_t)k / (uint32_t)len2);
+        int64_t at = o + s1 * c1[i];
+        double prod = sign * v1[i];
+        if (c2) {
+          const int64_t j = k - i * len2;
+          at += s2 * c2[j];
+          prod = prod * v2[j];
         }
-        const int32_t inv = sb.inv[sb_index(qq[0], qq[1], qq[2], qq[3], sb.dim_RR, sb.d)];
+        const int32_t inv = sb.inv[at];
         col = inv;
         v = prod;
         keep = inv >= 0 && inv <= r && fabs(prod) > kZero;

@@ -276,3 +276,22 @@ def test_assembly_list_lengths(left, right):
     sb.free()
     assert np.array_equal(row, orow) and np.array_equal(col, ocol)
     assert np.array_equal(val.view(np.int64), oval.view(np.int64))
+
+
+@pytest.mark.parametrize("copies", [5, 6, 11])
+def test_assembly_many_terms(copies):
+    """Term lists around and past the 64 terms that the assembly takes at a time (60 and 1, 72 and 1,
+    132 and 1), with terms that have no contribution in a row; identical to the oracle."""
+    from test_kron import _random_superblock
+    s = _random_superblock([6, 9, 5], [4, 10, 3], True, 13, True)
+    body, zero = s.terms[:-1][:12], s.terms[-1:]
+    terms = np.concatenate([body] * copies + [zero])
+    terms["coeff"][:-1] *= np.random.default_rng(2).uniform(0.5, 1.5, len(terms) - 1)
+    s.terms = terms
+    sb = D.Superblock(s)
+    sb.assemble(full=False)
+    row, col, val = sb.download_lower()
+    orow, ocol, oval = O.assemble(s)
+    sb.free()
+    assert np.array_equal(row, orow) and np.array_equal(col, ocol)
+    assert np.array_equal(val.view(np.int64), oval.view(np.int64))
