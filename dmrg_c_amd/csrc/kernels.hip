@@ -1167,18 +1167,19 @@ void Reduce::ensure(size_t blocks) {
   if (partial.count < blocks) partial.resize(blocks);
 }
 
-// Lanes per row of a CSR matrix.  A gather instruction touches fewer lines the more rows it
-// covers at like places, so few lanes win as long as the chip is full: 4 for rows of a dozen
-// entries, 16 above (8 would be a few percent faster still in large matrices, but every lane
-// then sums twice as long a chain, with that much more rounding).  Product and dot, microseconds,
-// at the old rule (a third of the row length, up to 64) and with 4 / 8 / 16 lanes: XXZ m = 162
-// (n = 23524, 164 a row) 21.9 and 13.9 / 12.6 / 13.2; Hubbard m = 250 (56244, 115) 43 and 20.3 /
-// 19.3 / 19.0; Hubbard m = 396 (144542, 186) 151 and 76 / 71 / 76; KLM m = 300 (287520, 131) 254 and
-// 114 / 107 / 120; KLM m = 60 (12870, 30) 7.4 and 6.1 / 6.3 / 6.4; XXZ m = 30 (790, 29) 5.6 and
-// 5.9 / 5.7 / 5.4; ED XXZ L = 20 (184756, 11) 14.0 and 10.5 / 14.2 / 21.8.
+// Lanes per row of a CSR matrix: a third of the mean row length, from 4 to 16.  A gather
+// instruction touches fewer lines the more rows it covers at like places, so few lanes win as
+// long as the chip is full.  Product and dot, microseconds, with 4 / 8 / 16 / 64 lanes (four loads
+// in flight): XXZ m = 162 (n = 23524, 164 a row) 14.9 / 12.9 / 13.3 / 16.6; Hubbard m = 250 (56244, 115)
+// 20.9 / 19.9 / 19.1 / 29.1; Hubbard m = 396 (144542, 186) 95 / 79 / 82 / 131; KLM m = 300 (287520, 131)
+// 140 / 123 / 124 / 206.  Shorter rows, 4 / 8 / 16 lanes: Hubbard m = 60 (3442, 28) 6.0 / 5.7 / 5.4;
+// banded, n = 200000, 14 a row 11.0 / 14.9 / 23.7, 24 a row 16.1 / 16.0 / 23.7; n = 20000, 20 a row
+// 8.8 / 6.1 / 6.9; ED XXZ L = 20 (184756, 11) 10.5 / 14.2 / 21.8.
 int pick_lanes(int32_t n, int64_t nnz) {
   const double avg = n > 0 ? (double)nnz / n : 0.0;
-  return avg < 12.0 ? 4 : 16;
+  int g = 4;
+  while (g < 16 && g * 3 < avg) g <<= 1;
+  return g;
 }
 
 void default_schedule(dmrgx_matrix &A) {

@@ -242,10 +242,10 @@ def test_gpu_sliced_ed_and_engine(lanes, cols16):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("k", [131, 350, 1000])
-def test_gpu_default_lanes_round_no_worse(k):
-    """The product under the default schedule against 80-bit sums.  Reference: 64 lanes a row,
-    each adding its k / 64 products one after another, then six levels of pairwise sums.  For products of
+@pytest.mark.parametrize("k,lanes", [(20, 8), (131, 64), (350, 64), (1000, 64)])
+def test_gpu_default_lanes_round_no_worse(k, lanes):
+    """The product under the default schedule against 80-bit sums.  Reference: a third of the row in
+    lanes, from 4 to 64, each adding its products one after another, then pairwise sums.  For products of
     variance 1 an addition whose result has variance c errs by 4.72e-17 sqrt(c) rms (a
     uniform error of half a unit in the last place over logarithmically spread mantissas), and the
     variances add up; 8 % are for the factors' fourth moments and the sample."""
@@ -260,7 +260,7 @@ def test_gpu_default_lanes_round_no_worse(k):
         err = (A.matvec(x) - exact).astype(float)
     finally:
         A.free()
-    per = np.bincount(np.arange(k) % 64, minlength=64)
-    c = (per * (per + 1) / 2).sum() + 6 * k
+    per = np.bincount(np.arange(k) % lanes, minlength=lanes)
+    c = (per * (per + 1) / 2).sum() + np.log2(lanes) * k
     rms = np.sqrt(np.mean(err * err))
     assert rms <= 1.08 * 4.72e-17 * np.sqrt(c), rms / (4.72e-17 * np.sqrt(c))
