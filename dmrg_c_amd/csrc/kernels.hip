@@ -1167,18 +1167,24 @@ void Reduce::ensure(size_t blocks) {
   if (partial.count < blocks) partial.resize(blocks);
 }
 
-// Lanes per row of a CSR matrix: a third of the mean row length, from 4 to 16.  A gather
+// Lanes per row of a CSR matrix: a third of the mean row length, from 4 to 16, and up to 64 while all
+// rows' lanes are no more than two wavefronts for each SIMD (kFewLanes).  A gather
 // instruction touches fewer lines the more rows it covers at like places, so few lanes win as
-// long as the chip is full.  Product and dot, microseconds, with 4 / 8 / 16 / 64 lanes (four loads
+// long as the chip is full; with few rows it is the length of a lane's chain of loads that
+// counts.  Product and dot, microseconds, with 4 / 8 / 16 / 64 lanes (four loads
 // in flight): XXZ m = 162 (n = 23524, 164 a row) 14.9 / 12.9 / 13.3 / 16.6; Hubbard m = 250 (56244, 115)
 // 20.9 / 19.9 / 19.1 / 29.1; Hubbard m = 396 (144542, 186) 95 / 79 / 82 / 131; KLM m = 300 (287520, 131)
 // 140 / 123 / 124 / 206.  Shorter rows, 4 / 8 / 16 lanes: Hubbard m = 60 (3442, 28) 6.0 / 5.7 / 5.4;
 // banded, n = 200000, 14 a row 11.0 / 14.9 / 23.7, 24 a row 16.1 / 16.0 / 23.7; n = 20000, 20 a row
-// 8.8 / 6.1 / 6.9; ED XXZ L = 20 (184756, 11) 10.5 / 14.2 / 21.8.
+// 8.8 / 6.1 / 6.9; ED XXZ L = 20 (184756, 11) 10.5 / 14.2 / 21.8.  Few rows, random columns, 16 / 32 /
+// 64 lanes: n = 500, 400 a row 7.8 / 6.4 / 5.7; 1000, 874 10.5 / 7.8 / 6.5; 2000, 201 6.6 / 6.1 / 6.0; 2000,
+// 1006 16.4 / 10.7 / 8.7; 4000, 100 6.2 / 6.2 / 6.6; 4000, 401 9.5 / 8.1 / 8.2; 8000, 200 8.7 / 9.6 / 10.6; 8000,
+// 1000 24.2 / 24.7 / 25.9.
+constexpr int64_t kFewLanes = 256 * 4 * 2 * 64;   // CUs x SIMDs x 2 wavefronts
 int pick_lanes(int32_t n, int64_t nnz) {
   const double avg = n > 0 ? (double)nnz / n : 0.0;
   int g = 4;
-  while (g < 16 && g * 3 < avg) g <<= 1;
+  while (g < 64 && g * 3 < avg && (g < 16 || 2 * g * (int64_t)n <= kFewLanes)) g <<= 1;
   return g;
 }
 
