@@ -566,7 +566,9 @@ int dmrgx_matrix_autotune(dmrgx_matrix *A, int32_t *lanes_out, int32_t *grid_out
   std::lock_guard<std::recursive_mutex> lk(api_mutex());
   return run_status([&] {
     TuneEnv env(A->n);
-    const int base = pick_lanes(A->n, A->nnz);
+    // around the row length's lanes rather than the default's: where a few rows are much longer
+    // than the mean, 64 lanes can be the fastest with any number of rows
+    const int base = lanes_by_length(A->n, A->nnz);
     const int caps[] = {1024, 2048, 4096, 8192, 16384, 0};
     const int g_lo = std::max(1, base / 16), g_hi = std::min(64, base * 2);
     struct Cand {

@@ -1026,6 +1026,7 @@ struct Reduce {              // deterministic two-kernel reduction workspace
   void ensure(size_t blocks);
 };
 
+int lanes_by_length(int32_t n, int64_t nnz);
 int pick_lanes(int32_t n, int64_t nnz);
 // CONVERGE_CHECK's product over caller-held device CSR arrays (default schedule of a matrix
 // of these dimensions), block partials at partial (residual_l1_default_blocks(n, nnz)

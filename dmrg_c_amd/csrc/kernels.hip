@@ -1167,6 +1167,14 @@ void Reduce::ensure(size_t blocks) {
   if (partial.count < blocks) partial.resize(blocks);
 }
 
+// A third of the mean row length in lanes, from 4 to 64.
+int lanes_by_length(int32_t n, int64_t nnz) {
+  const double avg = n > 0 ? (double)nnz / n : 0.0;
+  int g = 4;
+  while (g < 64 && g * 3 < avg) g <<= 1;
+  return g;
+}
+
 // Lanes per row of a CSR matrix: a third of the mean row length, from 4 to 16, and up to 64 while all
 // rows' lanes are no more than two wavefronts for each SIMD (kFewLanes).  A gather
 // instruction touches fewer lines the more rows it covers at like places, so few lanes win as
@@ -1182,9 +1190,8 @@ void Reduce::ensure(size_t blocks) {
 // 1000 24.2 / 24.7 / 25.9.
 constexpr int64_t kFewLanes = 256 * 4 * 2 * 64;   // CUs x SIMDs x 2 wavefronts
 int pick_lanes(int32_t n, int64_t nnz) {
-  const double avg = n > 0 ? (double)nnz / n : 0.0;
-  int g = 4;
-  while (g < 64 && g * 3 < avg && (g < 16 || 2 * g * (int64_t)n <= kFewLanes)) g <<= 1;
+  int g = lanes_by_length(n, nnz);
+  while (g > 16 && g * (int64_t)n > kFewLanes) g >>= 1;
   return g;
 }
 

@@ -283,3 +283,25 @@ def test_gpu_default_lanes(n, k, lanes):
         assert (abs(A.matvec(x) - (val * x[col]).sum(axis=1)) <= 2 * bound).all()
     finally:
         A.free()
+
+
+@pytest.mark.gpu
+def test_gpu_autotune_reaches_64_lanes():
+    """Rows of 100 entries and 16 of 6000: a product takes as long as the longest row, which 64 lanes
+    go through in half the passes of 32."""
+    import dmrg_c_amd as D
+    n = 6000
+    rng = np.random.default_rng(2)
+    length = np.where(np.arange(n) % 375 == 0, n, 100)
+    row = np.concatenate([[0], np.cumsum(length)])
+    col = np.concatenate([np.arange(n) if k == n else np.sort(rng.choice(n, k, replace=False)) for k in length])
+    val, x = rng.standard_normal(row[-1]), rng.standard_normal(n)
+    A = D.DeviceMatrix(row, col.astype(np.int32), val, sym=False)
+    try:
+        sched, _ = A.autotune()
+        assert sched[0] == 64, sched
+        y = np.add.reduceat(val * x[col], row[:-1])
+        bound = 2 * n * 2.0 ** -53 * np.add.reduceat(abs(val * x[col]), row[:-1])
+        assert (abs(A.matvec(x) - y) <= 2 * bound).all()
+    finally:
+        A.free()
