@@ -171,6 +171,7 @@ class Upload {
 struct dmrgx_matrix {
   int32_t n = 0;
   int64_t nnz = 0;
+  int64_t longest = 0;          // entries of the longest row, for a caller's CRS (0: not known)
   dmrgx::DevBuf<int64_t> row;
   dmrgx::DevBuf<int32_t> col;
   dmrgx::DevBuf<double> val;

@@ -949,10 +949,19 @@ __global__ __launch_bounds__(kBlock) void k_tri_count(int32_t n, const int64_t *
   }
 }
 
+// len[r] = entries of full row r; with longest set, *longest (zero before) becomes the largest.
 __global__ __launch_bounds__(kBlock) void k_row_len(int32_t n, const int64_t *trow,
-                                                    const unsigned *tcnt, int64_t *len) {
+                                                    const unsigned *tcnt, int64_t *len, int *longest) {
   const int32_t r = blockIdx.x * kBlock + threadIdx.x;
-  if (r < n) len[r] = (trow[r + 1] - trow[r]) + tcnt[r];
+  int l = 0;
+  if (r < n) {
+    len[r] = (trow[r + 1] - trow[r]) + tcnt[r];
+    l = (int)len[r];
+  }
+  if (!longest) return;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) l = max(l, __shfl_xor(l, off));
+  if ((threadIdx.x & 63) == 0) atomicMax(longest, l);
 }
 
 // exclusive scan of len[0..n) into out[0..n], 1024 elements per block
@@ -1198,6 +1207,15 @@ int pick_lanes(int32_t n, int64_t nnz) {
 void default_schedule(dmrgx_matrix &A) {
   A.lanes = pick_lanes(A.n, A.nnz);
   A.grid = kGridCap;
+  // A row that holds a good part of all entries, and several times the mean, is what a product waits
+  // for: more lanes and loads in flight for it.  Eight long rows among n = 100000 of 100 entries, 16
+  // lanes and this: 5000 long (1 / 2007 of the entries) 85 and 82 us, 10000 122 and 85, 20000
+  // 191 and 95; among n = 20000 of 100, 1200 long (1 / 1674) 19.5 and 19.8, 2500 26 and 20.
+  if (1500 * A.longest > A.nnz && A.longest * A.n > 4 * A.nnz) {
+    A.lanes = lanes_by_length(A.n, A.nnz);
+    A.load = kLoadDeep;
+    return;
+  }
   // eight loads in flight per lane where a lane has that many entries (in shorter rows the
   // positions past the end load the last entry again: ED XXZ L = 18, 10 a row, 7.1 against 6.3 us);
   // the value dictionary only where the tuner finds it faster (its table lookups cost more
@@ -1307,9 +1325,9 @@ int residual_l1_default_blocks(int32_t n, int64_t nnz) { return spmv_blocks(n, p
 
 void launch_residual_l1_into(int32_t n, int64_t nnz, const int64_t *row, const int32_t *col, const double *val,
                              const double *v, double eig, double *out, double *partial, hipStream_t s) {
-  // default_schedule's lanes and workgroups for a CSR matrix of these dimensions, so that the
-  // result equals launch_residual_l1 on a dmrgx_matrix of the same arrays bit for bit (the loads
-  // in flight do not change the order of the sums)
+  // default_schedule's lanes and workgroups for a CSR matrix of these dimensions (without a row that
+  // outweighs the others), so that the result equals launch_residual_l1 on a dmrgx_matrix of the
+  // same arrays bit for bit (the loads in flight do not change the order of the sums)
   apply_rows_into(n, pick_lanes(n, nnz), kGridCap, CsrRows<double, kLoadDeep>{row, col, val, nnz}, v,
                   EpiResidualL1{v, out, eig}, partial, s, 0, true, false);
 }
@@ -1874,16 +1892,16 @@ void launch_expand_lower(int32_t n, int64_t nnz_tri, const int64_t *trow, const 
   if (!cnt) {
     own.resize(n);
     tcnt.resize(n);
-    bad.resize(1);
+    bad.resize(2);   // the rows' faults, the longest full row
     HIPCHK(hipMemsetAsync(tcnt.p, 0, sizeof(unsigned) * n, s));
-    HIPCHK(hipMemsetAsync(bad.p, 0, sizeof(int), s));
+    HIPCHK(hipMemsetAsync(bad.p, 0, 2 * sizeof(int), s));
     k_tri_count<<<(n + kBlock / 64 - 1) / (kBlock / 64), kBlock, 0, s>>>(n, trow, tcol, own.p, tcnt.p, bad.p);
     HIPCHK(hipGetLastError());
     cnt = tcnt.p;
     badp = bad.p;
   }
   // row lengths and pointers before the structure check is read: one round trip for both
-  k_row_len<<<nb, kBlock, 0, s>>>(n, trow, cnt, len.p);
+  k_row_len<<<nb, kBlock, 0, s>>>(n, trow, cnt, len.p, bad.p ? bad.p + 1 : nullptr);
   HIPCHK(hipGetLastError());
   A.row.resize((size_t)n + 1);
   const int sb = (n + kScanChunk - 1) / kScanChunk;
@@ -1894,9 +1912,11 @@ void launch_expand_lower(int32_t n, int64_t nnz_tri, const int64_t *trow, const 
   HIPCHK(hipGetLastError());
   int64_t *h = reinterpret_cast<int64_t *>(ctx().host_stage(2));
   HIPCHK(hipMemcpyAsync(h, A.row.p + n, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-  HIPCHK(hipMemcpyAsync(h + 1, badp, sizeof(int), hipMemcpyDeviceToHost, s));
+  h[1] = 0;
+  HIPCHK(hipMemcpyAsync(h + 1, badp, sizeof(int) * (bad.p ? 2 : 1), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
-  const int hbad = *reinterpret_cast<const int *>(h + 1);
+  const int hbad = reinterpret_cast<const int *>(h + 1)[0];
+  A.longest = reinterpret_cast<const int *>(h + 1)[1];
   if (hbad & 1) throw Failure(DMRGX_ERR_NODIAG, "a row has no diagonal element as its last entry");
   if (hbad & 2) throw Failure(DMRGX_ERR_ARG, "lower-triangle CRS has a column outside [0,row)");
   const int64_t nnz = h[0];

@@ -305,3 +305,31 @@ def test_gpu_autotune_reaches_64_lanes():
         assert (abs(A.matvec(x) - y) <= 2 * bound).all()
     finally:
         A.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sym", [False, True], ids=["full", "lower"])
+def test_gpu_default_lanes_long_rows(sym):
+    """A row that holds a good part of all entries gets the lanes of the row length, however many rows
+    there are; one that does not, nothing."""
+    import dmrg_c_amd as D
+    import scipy.sparse as sp
+    n = 6000
+    rng = np.random.default_rng(4)
+    for long, want in ((0, 16), (200, 16), (n // 2, 64)):
+        i = np.repeat(np.arange(n), 60)
+        A = sp.coo_matrix((rng.standard_normal(60 * n), (i, rng.integers(0, n, 60 * n))), (n, n)).tolil()
+        A[n - 1, :long] = 1.0
+        A = sp.csr_matrix(A)
+        A = (A + A.T + sp.identity(n)).tocsr()
+        A.sort_indices()
+        B = sp.tril(A).tocsr() if sym else A
+        B.sort_indices()
+        M = D.DeviceMatrix(B.indptr.astype(np.int64), B.indices, B.data, sym=sym)
+        try:
+            assert M.schedule[0] == want and (M.schedule[2] == 2) == (want == 64), (long, M.schedule)
+            x = rng.standard_normal(n)
+            # a row's products and additions, whatever their order, on both sides
+            assert (abs(M.matvec(x) - A @ x) <= 4 * np.diff(A.indptr).max() * 2.0 ** -53 * (abs(A) @ abs(x))).all()
+        finally:
+            M.free()
