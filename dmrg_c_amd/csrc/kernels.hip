@@ -1216,11 +1216,14 @@ void default_schedule(dmrgx_matrix &A) {
     A.load = kLoadDeep;
     return;
   }
-  // eight loads in flight per lane where a lane has that many entries (in shorter rows the
-  // positions past the end load the last entry again: ED XXZ L = 18, 10 a row, 7.1 against 6.3 us);
-  // the value dictionary only where the tuner finds it faster (its table lookups cost more
-  // than the 4 bytes per entry they save on MI355X for the superblocks measured)
-  A.load = (double)A.nnz >= 12.0 * A.lanes * A.n ? kLoadDeep : 0;
+  // eight loads in flight per lane instead of four from 13 entries a lane; in shorter rows the
+  // positions past the end load the last entry again.  Product and dot, us, four and eight: ED XXZ
+  // L = 18, 10 a row, 6.3 and 7.1; 16 lanes, Hubbard m = 250 (115 a row) 19.1 and 19.6, KLM m = 300
+  // (131) 123.7 and 125.8, XXZ m = 162 (164) 13.3 and 13.7, Hubbard m = 396 (186) 81.6 and 80.3, n = 8000
+  // (200) 8.7 and 9.0, n = 16000 (401) 28.2 and 27.2, n = 32000 (399) 59.1 and 55.6; 64 lanes, n = 1000
+  // (874) 6.5 and 6.3.  The value dictionary only where the tuner finds it faster (its table lookups
+  // cost more than the 4 bytes per entry they save on MI355X for the superblocks measured).
+  A.load = (double)A.nnz >= 13.0 * A.lanes * A.n ? kLoadDeep : 0;
 }
 
 int spmv_blocks(int32_t n, int lanes, int grid_cap) {

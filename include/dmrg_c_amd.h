@@ -525,8 +525,8 @@ int dmrgx_spmv_host(const dmrgx_matrix *A, const double *x, double *y);
  * Bit 1, formats 1-2 against 0, format 4 against 3 and the sliced form's bit 0 never
  * change results; lanes, the sliced forms against the others, and CSR's bit 0 change
  * the summation order within a row, and cap and bit 2 the order of the dot products fused
- * into the solvers' products.  Defaults: lanes from the mean row length, cap 4096,
- * variant 2; dmrgx_matrix_autotune times every candidate on the device (product + fused
+ * into the solvers' products.  Defaults: lanes from the mean row length and the number of rows,
+ * cap 4096, variant 2 for long rows and 0 otherwise; dmrgx_matrix_autotune times every candidate on the device (product + fused
  * dot), then times the eight fastest as the solver runs them -- a Lanczos step and a CG
  * iteration with their fused vector kernels -- and keeps the fastest; *best_us_out is that
  * step-pair time.  Single and batched solves use the matrix's schedule. */

@@ -268,16 +268,18 @@ def test_gpu_default_lanes_round_no_worse(k, lanes):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,k,lanes", [(60, 11, 4), (60, 24, 8), (500, 48, 16), (500, 96, 32), (500, 400, 64), (2048, 97, 64),
-                                       (2049, 97, 32), (4096, 97, 32), (4097, 97, 16), (4097, 24, 8)])
+                                       (2049, 97, 32), (4096, 97, 32), (4097, 97, 16), (4097, 24, 8), (4097, 207, 16),
+                                       (4097, 208, 16)])
 def test_gpu_default_lanes(n, k, lanes):
-    """A third of the row length, up to 16 lanes, and up to 64 while there are few rows."""
+    """A third of the row length, up to 16 lanes, and up to 64 while there are few rows; eight loads in
+    flight from 13 entries a lane."""
     import dmrg_c_amd as D
     col = (np.arange(n)[:, None] * 7 % (n - k) + np.arange(k)).astype(np.int32)
     val = np.random.default_rng(n + k).standard_normal((n, k))
     x = np.random.default_rng(1).standard_normal(n)
     A = D.DeviceMatrix(np.arange(n + 1, dtype=np.int64) * k, col.ravel(), val.ravel(), sym=False)
     try:
-        assert A.schedule[0] == lanes
+        assert A.schedule == (lanes, 4096, 2 if k >= 13 * lanes else 0)
         # k products and k additions, whatever their order
         bound = 2 * k * 2.0 ** -53 * (abs(val) * abs(x[col])).sum(axis=1)
         assert (abs(A.matvec(x) - (val * x[col]).sum(axis=1)) <= 2 * bound).all()
