@@ -101,7 +101,10 @@ __global__ __launch_bounds__(64) void k_assemble(SbView sb, const int32_t *row_l
                                                  int32_t *scol = nullptr, double *sval = nullptr,
                                                  uint8_t *fitted = nullptr, unsigned *tcnt = nullptr,
                                                  int *bad = nullptr) {
-  __shared__ __align__(16) uint64_t key[CAP + 2];
+  constexpr bool kRank = CAP <= 256;   // sorted by rank, which reads the keys in pairs
+  constexpr int kKeys = kRank ? CAP + 2 : CAP;
+  static_assert((kKeys + CAP) * 8 <= 64 * 1024, "64 KiB of LDS a workgroup");
+  __shared__ __align__(16) uint64_t key[kKeys];
   __shared__ double val[CAP];
   const int lane = threadIdx.x;
   const int32_t item = blockIdx.x;
@@ -209,8 +212,8 @@ __global__ __launch_bounds__(64) void k_assemble(SbView sb, const int32_t *row_l
   const int64_t sbase = (int64_t)r * (CAP + 1);   // this row's scratch slot
   // key[0..m) in ascending order.  Short lists by rank (rank_keys); long ones by a bitonic sort
   // of key[0..P), P the next power of two (padding sorts last).
-  if constexpr (CAP <= 256) {
-    if (lane == 0 && (m & 1)) key[m] = ~0ull;   // the keys are read in pairs
+  if constexpr (kRank) {
+    if (lane == 0 && (m & 1)) key[m] = ~0ull;
     __syncthreads();
     if (m <= 64) rank_keys<1>(key, m);
     else if (m <= 128) rank_keys<2>(key, m);
@@ -317,11 +320,11 @@ __global__ __launch_bounds__(256) void k_inv_scatter(SbView sb, int32_t *inv) {
   inv[sb_index(sb.LL[r], sb.LR[r], sb.RR[r], sb.RL[r], sb.dim_RR, sb.d)] = r;
 }
 
-// List capacities of the three k_assemble variants: most rows fit the small one, whose 4 KiB
-// of LDS lets a CU hold as many rows as it has wave slots; longer rows are redone by the
+// List capacities of the three k_assemble variants: most rows fit the small one, whose 4112 bytes
+// of LDS let a CU hold as many rows as it has wave slots; longer rows are redone by the
 // larger variants.
-constexpr int kCapSmall = 256;   // 4 KiB of LDS per row
-constexpr int kCapMid = 1024;    // 16 KiB
+constexpr int kCapSmall = 256;   // one wavefront ranks four keys a lane
+constexpr int kCapMid = 1024;    // 16 KiB of LDS per row
 constexpr int kCapLarge = 4096;  // 64 KiB
 // Device scratch the count pass may use to keep its rows' entries (n * (kCapSmall + 1) * 12
 // bytes: 0.45 GB at n = 144542, 6.1 GB at n = 1993680; held only during the assembly).

@@ -263,10 +263,12 @@ def test_expand_tail_lengths():
         assert np.array_equal(g, r)
 
 
-@pytest.mark.parametrize("left,right", [([1], [1]), ([30, 33], [31, 35]), ([60, 70], [66, 64]), ([120, 140], [4, 3])])
+@pytest.mark.parametrize("left,right", [([1], [1]), ([30, 33], [31, 35]), ([60, 70], [66, 64]), ([120, 140], [4, 3]),
+                                        ([2, 1021], [1, 1]), ([3, 1100], [1, 2])])
 def test_assembly_list_lengths(left, right):
-    """Rows of 1 to 266 entries: contribution lists on both sides of every length at which the
-    assembly's sort changes over, and past the short list's capacity; identical to the oracle."""
+    """Rows of 1 to 1100 entries: contribution lists on both sides of every length at which the
+    assembly's sort changes over, and past the short list's capacity and the middle one's (whose rows
+    go to the variant with 64 KiB of LDS); identical to the oracle."""
     from test_kron import _random_superblock
     s = _random_superblock(left, right, True, 11)
     sb = D.Superblock(s)
