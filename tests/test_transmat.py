@@ -97,11 +97,12 @@ def call(fn, M1, M2, M3, n1, n2, n3, k, out_cap=None, work_cap=None, work_out=No
     return orow, ocol[:nnz], oval[:nnz]
 
 
-def random_case(seed, n1, n2, n3, k, density=0.2):
+def random_case(seed, n1, n2, n3, k, density=0.2, dup=False):
     rng = np.random.default_rng(seed)
     M1 = rand_crs(rng, n1, n2, density, shuffle=True, dup=True)
     M2 = rand_crs(rng, n2, n3, density, shuffle=True, tiny=True)
-    c3 = rand_crs(rng, k, n3, density)   # CCS of M3 = CRS of its transpose
+    # CCS of M3 = CRS of its transpose; with dup a row out of order and twice in every column
+    c3 = rand_crs(rng, k, n3, density, shuffle=dup, dup=dup)
     return M1, M2, c3, (n1, n2, n3, k)
 
 
@@ -127,6 +128,13 @@ def truncation_case():
 CASES = {f"random{s}": random_case(s, *dims) for s, dims in enumerate([(7, 9, 11, 5), (40, 60, 50, 30),
                                                                         (1, 1, 1, 1), (64, 300, 200, 17)])}
 CASES["truncation"] = truncation_case()
+# the device's result: 63, 64 and 65 columns (its compaction takes 64 at a time), 257 and 400 (more
+# than one workgroup a row); 332 and 333 rows of 65 columns (261640 bytes come back in one copy, 262428
+# in three, the line is 256 KiB); repeated rows in M3's columns, of which the last value counts
+CASES.update({f"k{k}_{n1}": random_case(20 + k, n1, 40, 30, k) for n1, k in ((9, 63), (10, 64), (11, 65), (20, 257), (90, 257),
+                                                                        (120, 400))})
+CASES.update({f"result{n1}": random_case(n1, n1, 50, 40, 65) for n1 in (332, 333)})
+CASES.update({f"dup{k}": random_case(30 + k, 12, 40, 150, k, dup=True) for k in (5, 70)})
 
 
 @pytest.mark.parametrize("name", list(CASES))
@@ -196,10 +204,10 @@ def _cap_boundaries():
     return w_nnz - int(w_last), o_nnz - int(o_last), w_nnz, o_nnz
 
 
-def _run_child(which, out_cap, work_cap):
+def _run_child(which, out_cap, work_cap, case=CAP_CASE):
     code = (f"import sys; sys.path[:0] = [{os.path.dirname(os.path.abspath(__file__))!r}, {REPO!r}]\n"
             "import ctypes as C, test_transmat as T\n"
-            f"M1, M2, M3, dims = T.CASES[{CAP_CASE!r}]\n"
+            f"M1, M2, M3, dims = T.CASES[{case!r}]\n"
             + ("fn = C.CDLL(T.REF_LIB).CRS_CRS_CCS_PRODUCT\n" if which == "ref"
                else "import dmrg_c_amd as D; fn = D.lib().CRS_CRS_CCS_PRODUCT\n")
             + f"T.call(fn, M1, M2, M3, *dims, out_cap={out_cap}, work_cap={work_cap})\n")
@@ -233,3 +241,16 @@ def test_device_capacity_rule():
     for out_cap, work_cap, exits in _cap_cases():
         print(f"crs_crs_ccs capacity out={out_cap} work={work_cap}", flush=True)
         assert (_run_child("dev", out_cap, work_cap) != 0) == exits, (out_cap, work_cap, exits)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", [CAP_CASE, "k400_120"])
+def test_device_out_capacity(name):
+    """The same rule on Out with the oracle's result in the reference's place, for a result that
+    comes back in one copy and one that does not."""
+    M1, M2, M3, (n1, n2, n3, k) = CASES[name]
+    row, col, _ = oracle(M1, M2, M3, n1, n2, n3, k)
+    before = int(row[n1]) - int(row[n1] > row[n1 - 1] and col[-1] == k - 1)
+    for cap, exits in ((before, True), (before + 1, False)):
+        print(f"crs_crs_ccs capacity {name} out={cap}", flush=True)
+        assert (_run_child("dev", cap, 10 ** 6, name) != 0) == exits, (cap, exits)
