@@ -736,9 +736,10 @@ class KronOperator:
         check(L.dmrgx_kron_info(h, C.byref(n), C.byref(ns), C.byref(nc), C.byref(fl)))
         self.n, self.sectors, self.coupling_terms, self.flops = n.value, ns.value, nc.value, fl.value
 
-    VARIANTS = 16
+    VARIANTS = 16   # numbers accepted; 3 to 15 mean 1
 
     def set_kernel(self, variant: int):
+        """Product kernel: 0 with 16 x 16 output tiles, 2 with 32 x 32, 1 (default) by size."""
         check(lib().dmrgx_kron_set_kernel(self.handle, variant))
 
     def autotune(self):

@@ -970,7 +970,8 @@ struct KronView {
 constexpr int kKronShapes = 2;
 inline constexpr int kKronTile[kKronShapes] = {16, 32};
 // Product kernels a caller can choose (dmrgx_kron_set_kernel): 0 and 2 fix the shape 16 x 16 and
-// 32 x 32, the default and every other number take it by size (kron_shape_rule).
+// 32 x 32, the default 1 takes it by size (kron_shape_rule).  3 to 15 have no kernel of their own;
+// they are accepted, as the default, for programs that kept a number.
 constexpr int kKronVariants = 16;
 constexpr int kKronDefault = 1;
 struct KronDev {

@@ -665,9 +665,9 @@ int dmrgx_superblock_kron(const dmrgx_superblock *S, dmrgx_kron **out);
 /* dimension, sectors, coupling terms, floating-point operations of the dense products per
  * product (any pointer may be null) */
 int dmrgx_kron_info(const dmrgx_kron *K, int32_t *n, int32_t *sectors, int32_t *coupling_terms, double *flops);
-/* product kernel, 0 to 15: 0 with 16 x 16 output tiles, 2 with 32 x 32, every other number
- * (default 1) the one of the two that the superblock's size calls for.  The results agree to
- * rounding between them. */
+/* product kernel: 0 with 16 x 16 output tiles, 2 with 32 x 32, 1 (default) the one of the two that
+ * the superblock's size calls for; 3 to 15 have no kernel of their own and mean 1, other numbers
+ * are refused.  The results agree to rounding between them. */
 int dmrgx_kron_set_kernel(dmrgx_kron *K, int32_t variant);
 /* times the kernels (5 products each after one warm-up) and keeps the fastest; the default
  * (variant 1) stays unless another is more than 2 % faster */
