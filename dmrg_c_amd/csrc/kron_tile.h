@@ -57,7 +57,7 @@ struct KronFrag {
 // kron_slab: no clamping at the edge).
 //
 // Measured (MI355X, KLM m = 799: 3.23 GFLOP a product, 2133 tiles of 32 x 32): 88 us with the Lanczos
-// epilogue and 72 with CG's, of which the matrix cores are busy 46; 64 x 64 LDS-staged tiles took 86 us
+// epilogue and 75 with CG's, of which the matrix cores are busy 46; 64 x 64 LDS-staged tiles took 86 us
 // and the epilogue's own kernel 14 to 25 more, with the coupling terms on a side stream.  Whole
 // solves by tile: 32 x 32 83 ms, 32 x 64 84 to 87 ms, 64 x 64 101 to 107 ms.  Hubbard m = 396
 // (68 MFLOP, 641 tiles of 16 x 16): 9 us against 30, most of it latency.
@@ -68,7 +68,7 @@ template <int B, class Epi>
 __global__ __launch_bounds__(256, 4) void k_kron(KronView kv, const double *__restrict__ x, Epi epi, double *partial) {
   if (epi.skip()) return;
   constexpr bool kStaged = B > 1;
-  constexpr int kRow = 18;   // doubles per staged row: 16-byte aligned, no bank conflicts
+  constexpr int kRow = 18;   // doubles per staged row: 16-byte aligned, few bank conflicts (1.5 cycles an access)
   constexpr int E = 4 * B * B, NE = B * B;   // a wavefront's elements per lane, this one's finished
   constexpr int kStage = kStaged ? 16 * B * kRow : 0;
   constexpr int kLds = 2 * kStage > E * 64 ? 2 * kStage : E * 64;
